@@ -1105,11 +1105,20 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
     const int g32 = c->precision != RP_PREC_FP64 && waves == 8 && sp.pipelined == 2 && !c->k.soft && !c->counting &&
                     c->k.kind == RP_SHAPE_SPHEROCYLINDER && !g.allPairs ? c->precision : 0;
     if (g32) g32Limits(c, g, sp.g32Lim);
-    const double perEntry =
-        (double)(sweep_lds_bytes(c->k.kind, 1024, waves, g32) - sweep_lds_bytes(c->k.kind, 0, waves, g32)) / 1024.0;
-    const size_t fixed = sweep_lds_bytes(c->k.kind, 0, waves, g32);
+    {
+        // the contact distance raised by a relative 1e-7 and by 1e-11 of the box's extent: the coordinates' rounding, and
+        // that of the sums it propagates through, is below 1e-13 of the extent
+        double extent = 0;
+        for (int i = 0; i < 9; i++) extent += std::fabs(g.dims[i]);
+        const double d = std::sqrt(c->k.contact2) * (1 + 1e-7) + 1e-11 * extent;
+        sp.skip2 = d * d;
+    }
+    const bool lean = sweep_is_lean(c->k, waves, sp.pipelined, c->counting && !c->k.soft);
+    const size_t fixed = sweep_lds_bytes(c->k.kind, 0, waves, g32, lean);
+    const double perEntry = (double)(sweep_lds_bytes(c->k.kind, 1024, waves, g32, lean) - fixed) / 1024.0;
     int maxCap = (int)((double)(c->ldsLimit - fixed) / perEntry) / 64 * 64;
     sp.cap = std::max(64, std::min(cap, maxCap));
+    if (lean) sp.cap = std::min(sp.cap, sweep_lean_cap());
     // workgroups that read their stencil from HBM so far (hCounters as of the last read)
     if (!c->pairCapOff && c->blocksAtRead >= 10000 && c->hCounters[CNT_UNSTAGED_BLOCKS] * 100 > c->blocksAtRead)
         c->pairCapOff = true;
@@ -1514,7 +1523,9 @@ int runReplicas(rp_ctx *const *ctxs, size_t n, size_t nCycles, bool adapt, rp_co
                         mem.hTable[entries++] = sp;
                         pg.blocks += (unsigned)(sp.na[0] * sp.na[1] * sp.na[2]);
                         mem.hFirst[++firsts] = (int)pg.blocks;
-                        pg.lds = std::max(pg.lds, sweep_lds_bytes(sp.k.kind, sp.cap, plans[i].waves, plans[i].g32));
+                        pg.lds = std::max(pg.lds, sweep_lds_bytes(sp.k.kind, sp.cap, plans[i].waves, plans[i].g32,
+                                                                       sweep_is_lean(sp.k, plans[i].waves, sp.pipelined,
+                                                                                     sp.counting != 0)));
                     }
                     firsts++;
                     groups.push_back(pg);
@@ -2122,7 +2133,13 @@ void rp_destroy(rp_ctx *c) {
                          (unsigned long long)ph[RP_PHASE_BLOCKS], ph[RP_PHASE_LAST] / perUs, khz,
                          sweep_occupancy(c->shape.kind, c->tstats.sweep_cap ? (int)c->tstats.sweep_cap : 64,
                                          c->tstats.sweep_waves ? (int)c->tstats.sweep_waves : 4));
-            if (ph[RP_PHASE_GROUPS]) {
+            if (ph[RP_PHASE_GROUPS] && ph[RP_PHASE_TOP] == 0) {
+                std::fprintf(stderr,
+                             "speculative sweep per workgroup (us): first scan %.2f, rescans %.2f, decisions %.2f; %.2f "
+                             "accepted moves, %.2f rescans\n",
+                             ph[RP_PHASE_PLAN] / b / perUs, ph[RP_PHASE_SCAN] / b / perUs,
+                             ph[RP_PHASE_DECIDE] / b / perUs, ph[RP_PHASE_GROUPS] / b, ph[RP_PHASE_REPLANS] / b);
+            } else if (ph[RP_PHASE_GROUPS]) {
                 const double ng = (double)ph[RP_PHASE_GROUPS];
                 std::fprintf(stderr,
                              "grouped sweep per group (us): loop top %.3f, planner busy %.3f, tester busy %.3f "

@@ -90,6 +90,7 @@ struct SweepParams {
     // range2 upper} bounds of the FP32 guard bands, s = 0 for cells whose stencil was staged translated (no wrapped
     // particle), s = 1 otherwise (positions and image translations up to a box length from the centre).
     float g32Lim[2][4];
+    double skip2;        // speculative sweep: a squared distance bound above which segments certainly do not touch
     double mlpInvRange;  // candidate pairs of the learned ordering: 1 / total interaction range (feature scale)
 };
 
@@ -246,7 +247,10 @@ int sweep_occupancy(int kind, int cap, int waves);
 // records the largest FP32 error and any class mismatch (counters CNT_G32_*).  g32 > 0 needs eight wavefronts, the
 // grouped launch and a hard sphere or spherocylinder.
 hipError_t launch_sweep(hipStream_t s, const SweepParams &sp, int waves, Timed t = {}, int g32 = 0);
-size_t sweep_lds_bytes(int kind, int cap, int waves, int g32 = 0);
+size_t sweep_lds_bytes(int kind, int cap, int waves, int g32 = 0, bool lean = false);
+// Whether a (non-fix) sweep of this launch shape runs the speculative kernel.
+int sweep_lean_cap();  // stencil entries it can stage at most
+bool sweep_is_lean(const PairConsts &k, int waves, int pipelined, bool counting);
 // The kernel launch_sweep(sp, waves, g32) would run, as a key shared by the packings one batched launch may hold, or
 // -1 for the sweeps that run one packing per launch (soft, overlap counting, orientation fix, polyspheres, traced).
 int sweep_batch_key(const SweepParams &sp, int waves, int g32);

@@ -61,6 +61,25 @@ __device__ __forceinline__ void bin_position(const Grid &g, const V3 &pos, int c
     }
 }
 
+// bin_position in a shifted grid (exact = 0) whose box inverse and origin shift the caller keeps elsewhere (in LDS:
+// the sweep's planning lanes then hold none of it in scalar registers).
+__device__ __forceinline__ void bin_shifted(const double *inv, const double *shift, const int n[3], const V3 &pos, int c[3],
+                                            unsigned &wbits) {
+    const V3 rel = mulv(inv, pos);
+    const double r[3] = {rel.x, rel.y, rel.z};
+    wbits = 0;
+    for (int d = 0; d < 3; d++) {
+        const int w = r[d] < shift[d] ? 1 : 0;
+        const double y = (r[d] - shift[d]) + (w ? 1.0 : 0.0);
+        int cc = (int)(y * (double)n[d]);
+        if (w) cc = n[d] - 1;
+        wbits |= (unsigned)w << d;
+        if (cc < 0) cc = 0;
+        if (cc > n[d] - 1) cc = n[d] - 1;
+        c[d] = cc;
+    }
+}
+
 __device__ __forceinline__ int cell_index(const Grid &g, int cx, int cy, int cz) {
     return cx + g.n[0] * (cy + g.n[1] * cz);
 }
@@ -681,9 +700,16 @@ __device__ __forceinline__ void build_stencil(const Grid &g, int cx, int cy, int
     for (int slot = threadIdx.x; slot < ncells; slot += blockDim.x)
         stencil_table(g, cx, cy, cz, slot, half, s_start, s_base, s_ecode, byShell);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        s_start[0] = 0;
-        for (int q = 1; q <= ncells; q++) s_start[q] += s_start[q - 1];
+    if (threadIdx.x < WAVE) {
+        // prefix sums of the counts, a wavefront's worth at a time
+        int base = 0;
+        for (int q0 = 0; q0 < ncells; q0 += WAVE) {
+            const int q = q0 + (int)threadIdx.x;
+            const int sum = base + wave_inclusive_scan(q < ncells ? s_start[q + 1] : 0);
+            if (q < ncells) s_start[q + 1] = sum;
+            base = __shfl(sum, WAVE - 1);
+        }
+        if (threadIdx.x == 0) s_start[0] = 0;
     }
     __syncthreads();
 }
@@ -1266,12 +1292,14 @@ hipError_t launch_type_counts(hipStream_t s, const Proposals &pr, size_t total, 
 
 // LDS of one sweep workgroup: the stencil (cap entries), the ambiguous-candidate queues (cap + 64*waves ints),
 // own orientations, one batch of proposals and the translation table.
-// The guarded FP32 scan adds the FP32 stencil positions (3 x cap floats) and the FP32 translation table (81 floats).
-size_t sweep_lds_bytes(int kind, int cap, int waves, int g32) {
+// lean: the speculative sweep's own layout (spec_lds_bytes).
+size_t spec_lds_bytes(int kind, int cap, int waves, int g32);
+
+size_t sweep_lds_bytes(int kind, int cap, int waves, int g32, bool lean) {
+    if (lean) return spec_lds_bytes(kind, cap, waves, g32);
     const int queueInts = max(cap + WAVE * waves, (waves - 1) * GROUPED_QUEUE);
     return stencil_lds_bytes(kind, cap) + sizeof(int) * queueInts +
-           sizeof(double) * (9 * OWN_CAP + 12 * MOVE_CHUNK + 81 + SWEEP_AUX) + sizeof(int) * (MOVE_CHUNK + SWEEP_AUX_I) +
-           (g32 ? sizeof(float) * (3 * (size_t)cap + 81) : 0);
+           sizeof(double) * (9 * OWN_CAP + 12 * MOVE_CHUNK + 81 + SWEEP_AUX) + sizeof(int) * (MOVE_CHUNK + SWEEP_AUX_I);
 }
 
 __device__ __forceinline__ void flush_counters(const SweepParams &P, int cell, unsigned long long accepted, int moves,
@@ -1696,7 +1724,8 @@ __device__ __forceinline__ int poly_count(const PairConsts &k, const double *sBe
 
 template <int KIND, int WAVES>
 __device__ __forceinline__ void sweep_cell_unstaged(const SweepParams &P, const Stencil &S, double *pt, double *pR, int *pk,
-                                    const double *sT, int cell, int own0, int nOwn, int total) {
+                                    const double *sT, int cell, int own0, int nOwn, int total, const double *dims,
+                                    const double *inv, const double *shift) {
     constexpr int NT = WAVE * WAVES;
     const Grid &g = P.g;
     const int tid = threadIdx.x;
@@ -1724,11 +1753,11 @@ __device__ __forceinline__ void sweep_cell_unstaged(const SweepParams &P, const 
             V3 npos = pos;
             if (!P.fixMode) {
                 V3 t = v3(pt[mi], pt[MOVE_CHUNK + mi], pt[2 * MOVE_CHUNK + mi]);
-                npos = translate_wrapped(g.dims, g.inv, pos, t);
+                npos = translate_wrapped(dims, inv, pos, t);
             }
             int nc[3];
             unsigned nw;
-            bin_position(g, npos, nc, nw);
+            bin_shifted(inv, shift, g.n, npos, nc, nw);
             if (cell_index(g, nc[0], nc[1], nc[2]) != cell) {
                 leftCell++;
                 continue;
@@ -1860,11 +1889,10 @@ __device__ __forceinline__ int wrap_code(unsigned nw) {
 
 // Planner wavefront: lane t < gs plans move m0 + t into plan slot t; then lanes 0-5 test the trial poses against
 // each other (bit 4k + i: move k's trial pose overlaps move i's trial pose, i < k).
-// With G32 the plan also carries the trial position relative to o in FP32 (three floats in doubles 22-23).
-template <int KIND, bool TRANSLATED, bool G32 = false>
+template <int KIND, bool TRANSLATED>
 __device__ __forceinline__ void plan_group(const SweepParams &P, const Stencil &S, const double *oo, const double *pt,
                                            const double *pR, const int *pk, const double *sT, int m0, int gs,
-                                           int cell, double *plan, int *planI, V3 o = V3{}) {
+                                           int cell, double *plan, int *planI) {
     const Grid &g = P.g;
     const int lane = threadIdx.x & (WAVE - 1);
     unsigned byte = 0;
@@ -1896,12 +1924,6 @@ __device__ __forceinline__ void plan_group(const SweepParams &P, const Stencil &
             q[12] = f.a;
         }
         for (int c = 0; c < 9; c++) q[13 + c] = NO[c];
-        if (G32) {
-            float *qf = reinterpret_cast<float *>(q + 22);
-            qf[0] = (float)(npos.x - o.x);
-            qf[1] = (float)(npos.y - o.y);
-            qf[2] = (float)(npos.z - o.z);
-        }
         planI[lane] = kIdx;
     }
     unsigned word = 0;
@@ -1935,17 +1957,11 @@ __device__ __forceinline__ void plan_group(const SweepParams &P, const Stencil &
     }
 }
 
-// G32 = 1: the stencil scan classifies each (candidate, move) pair from the FP32 squared centre distance (positions
-// relative to o); a pair whose FP32 value lies inside a guard band around contact^2 or range^2 (g32Lim) is decided
-// by the FP64 distance, the same value the FP64 scan computes, so every decision equals the FP64 sweep's.  The
-// bands are wider than the largest FP32 error the positions' magnitudes allow.  G32 = 2 also evaluates every pair in
-// FP64 and records the largest FP32 error and any class that differs (none may).
-template <int KIND, int WAVES, bool TRANSLATED, int G32 = 0>
+template <int KIND, int WAVES, bool TRANSLATED>
 __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const Stencil &S, double *oo, double *pt,
                                                    double *pR, int *pk, int *queue, const double *sT, double *plans,
                                                    int *plansI, int *hitWords, int own0, int nOwn, int total, int cell,
-                                                   unsigned long long *clk, float *Sf = nullptr,
-                                                   const float *sTf = nullptr, V3 o = V3{}) {
+                                                   unsigned long long *clk) {
     constexpr int NTT = WAVE * (WAVES - 1);
     // a tester's queue: entries [0, GQ - WAVE), then one discard slot per lane for lanes with nothing to queue; a
     // slot adds at most GROUP * WAVE entries, so the queue is drained once it holds more than QFLUSH
@@ -1960,9 +1976,6 @@ __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const S
     int *discard = myQueue + (GQ - WAVE) + lane;
     unsigned long long accepted = 0, leftCell = 0, tests = 0;
     unsigned long long tBusy = 0, tDecide = 0, tTop = 0, tPassB = 0, nGroups = 0, nReplans = 0;  // phase timers
-    unsigned g32Guard = 0, g32Mismatch = 0;  // guarded FP32 scan statistics of this lane
-    unsigned long long g32Pairs = 0;         // pairs classified by this workgroup (one lane keeps the count)
-    float g32Err = 0.f;
     const int moves = P.moves > 0 ? P.moves : nOwn * P.mult;
     const int pbase = P.moves > 0 ? cell * P.moves : own0 * P.mult;
     // issue priority: the planner and the testers with an extra slot bound each group's time
@@ -1991,7 +2004,7 @@ __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const S
         }
         int gidx = 0;
         int gs = __builtin_amdgcn_readlane(groups, 0) >> 8;
-        if (planner) plan_group<KIND, TRANSLATED, G32 != 0>(P, S, oo, pt, pR, pk, sT, 0, gs, cell, plans, plansI, o);
+        if (planner) plan_group<KIND, TRANSLATED>(P, S, oo, pt, pR, pk, sT, 0, gs, cell, plans, plansI);
         __syncthreads();
         for (; gidx < ngroups; gidx++) {
             const unsigned long long tgTop = clk ? wall_clock64() : 0;
@@ -2005,16 +2018,10 @@ __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const S
             const int gsNext = gidx + 1 < ngroups ? __builtin_amdgcn_readlane(groups, gidx + 1) >> 8 : 0;
             int kIdx[GROUP];
             V3 npos[GROUP];
-            float fm[GROUP][3];  // G32: trial positions relative to o
 #pragma unroll
             for (int k = 0; k < GROUP; k++) {
                 kIdx[k] = k < gs ? __builtin_amdgcn_readlane(pkv, m0 + k) : -1;
-                if (G32) {
-                    const float *qf = reinterpret_cast<const float *>(plan + k * PLAN_D + 22);
-                    for (int c = 0; c < 3; c++) fm[k][c] = k < gs ? qf[c] : 0.f;
-                } else {
-                    npos[k] = k < gs ? v3(plan[k * PLAN_D], plan[k * PLAN_D + 1], plan[k * PLAN_D + 2]) : v3(0, 0, 0);
-                }
+                npos[k] = k < gs ? v3(plan[k * PLAN_D], plan[k * PLAN_D + 1], plan[k * PLAN_D + 2]) : v3(0, 0, 0);
             }
             const unsigned newHit = (unsigned)__builtin_amdgcn_readfirstlane(planI[5]);
             const unsigned word = (unsigned)__builtin_amdgcn_readfirstlane(planI[6]);  // nw | inside << 3 per move
@@ -2031,8 +2038,8 @@ __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const S
             const unsigned long long tg0 = clk ? wall_clock64() : 0;
             if (planner) {
                 if (gsNext)
-                    plan_group<KIND, TRANSLATED, G32 != 0>(P, S, oo, pt, pR, pk, sT, m1, gsNext, cell,
-                                                           plans + nbuf * GROUP * PLAN_D, plansI + nbuf * GPLAN_I, o);
+                    plan_group<KIND, TRANSLATED>(P, S, oo, pt, pR, pk, sT, m1, gsNext, cell,
+                                                  plans + nbuf * GROUP * PLAN_D, plansI + nbuf * GPLAN_I);
                 if (lane == 0) hitWords[nbuf] = 0;
             } else {
                 // 5 bits per move: bits 0-3 overlap with group particle i's current pose, bit 4 with a particle
@@ -2051,74 +2058,25 @@ __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const S
                     for (int i = 0; i < GROUP; i++) groupBit = jj == kIdx[i] ? 1u << i : groupBit;
                     // the moves' distances first, as independent chains, then their hit bits and queue entries
                     double d2[GROUP];
-                    float d2f[GROUP];
-                    if (G32) {
-                        const float fj[3] = {Sf[jj], Sf[P.cap + jj], Sf[2 * P.cap + jj]};
+                    const V3 p2 = v3(S.x[jj], S.y[jj], S.z[jj]);
 #pragma unroll
-                        for (int k = 0; k < GROUP; k++) {
-                            float q[3] = {fj[0], fj[1], fj[2]};
-                            if (!TRANSLATED) {
-                                const unsigned wk = (word >> (4 * k + 3)) & 1 ? (word >> (4 * k)) & 7 : 0u;
-                                const int kx = (code & 3) - 1 - (int)(wk & 1), ky = ((code >> 2) & 3) - 1 - (int)((wk >> 1) & 1),
-                                          kz = ((code >> 4) & 3) - 1 - (int)((wk >> 2) & 1);
-                                const int t = 3 * ((kx + 1) * 9 + (ky + 1) * 3 + (kz + 1));
-                                for (int c = 0; c < 3; c++) q[c] = q[c] + sTf[t + c];
-                            }
-                            const float dx = q[0] - fm[k][0], dy = q[1] - fm[k][1], dz = q[2] - fm[k][2];
-                            d2f[k] = (dx * dx + dy * dy) + dz * dz;
+                    for (int k = 0; k < GROUP; k++) {
+                        V3 q2 = p2;
+                        if (!TRANSLATED) {
+                            // a move that leaves the cell is not tested; its wrap bits are zeroed so that the
+                            // translation index stays inside the 27-entry table
+                            const unsigned wk = (word >> (4 * k + 3)) & 1 ? (word >> (4 * k)) & 7 : 0u;
+                            q2 = add(p2, image_translation(sT, code, wk & 1, (wk >> 1) & 1, (wk >> 2) & 1));
                         }
-                    } else {
-                        const V3 p2 = v3(S.x[jj], S.y[jj], S.z[jj]);
-#pragma unroll
-                        for (int k = 0; k < GROUP; k++) {
-                            V3 q2 = p2;
-                            if (!TRANSLATED) {
-                                // a move that leaves the cell is not tested; its wrap bits are zeroed so that the
-                                // translation index stays inside the 27-entry table
-                                const unsigned wk = (word >> (4 * k + 3)) & 1 ? (word >> (4 * k)) & 7 : 0u;
-                                q2 = add(p2, image_translation(sT, code, wk & 1, (wk >> 1) & 1, (wk >> 2) & 1));
-                            }
-                            const V3 d = sub(q2, npos[k]);
-                            d2[k] = dot(d, d);
-                        }
+                        const V3 d = sub(q2, npos[k]);
+                        d2[k] = dot(d, d);
                     }
 #pragma unroll
                     for (int k = 0; k < GROUP; k++) {
                         if (k < gs && ((word >> (4 * k + 3)) & 1)) {  // moves leaving the cell are rejected
                             const bool other = valid && jj != kIdx[k];
-                            bool close, within;
-                            if (G32) {
-                                const float *lim = P.g32Lim[TRANSLATED ? 0 : 1];
-                                const float x = d2f[k];
-                                close = x < lim[0];
-                                within = x < lim[2];
-                                const bool guard = (x >= lim[0] && x < lim[1]) || (KIND == 1 && x >= lim[2] && x < lim[3]);
-                                if (guard || G32 == 2) {
-                                    // the FP64 squared distance of the FP64 scan (rare outside verify mode)
-                                    const double *qn = plan + k * PLAN_D;
-                                    V3 q2 = v3(S.x[jj], S.y[jj], S.z[jj]);
-                                    if (!TRANSLATED) {
-                                        const unsigned wk = (word >> (4 * k)) & 7;
-                                        q2 = add(q2, image_translation(sT, code, wk & 1, (wk >> 1) & 1, (wk >> 2) & 1));
-                                    }
-                                    const V3 d = sub(q2, v3(qn[0], qn[1], qn[2]));
-                                    const double e2 = dot(d, d);
-                                    const bool c64 = e2 < P.k.contact2, w64 = e2 < P.k.range2;
-                                    if (G32 == 2 && other) {
-                                        g32Err = fmaxf(g32Err, (float)fabs((double)x - e2));
-                                        if (!guard && (c64 != close || (KIND == 1 && !c64 && w64 != within)))
-                                            g32Mismatch++;
-                                    }
-                                    if (guard) {
-                                        close = c64;
-                                        within = w64;
-                                        g32Guard += other ? 1u : 0u;
-                                    }
-                                }
-                            } else {
-                                close = d2[k] < P.k.contact2;
-                                within = d2[k] < P.k.range2;
-                            }
+                            const bool close = d2[k] < P.k.contact2;
+                            const bool within = d2[k] < P.k.range2;
                             hitAll |= other && close ? groupBit << (5 * k) : 0u;
                             if (KIND == 1) {
                                 const bool amb = other && !close && within;
@@ -2182,8 +2140,6 @@ __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const S
             accepted += (unsigned long long)__popc(acc);
             leftCell += (unsigned long long)(gs - __popc(insideMask));
             tests += (unsigned long long)total * (unsigned long long)__popc(insideMask);
-            if (G32 && !planner && lane == 0 && wave == 1)  // pairs the scan classified (the moved particles' own
-                g32Pairs += (unsigned long long)(total - 1) * (unsigned long long)__popc(insideMask);  // excluded)
             const bool replan = (acc & nextUses) != 0;
             // accepted poses into this wavefront's view of the staged copy, one lane per component; LDS accesses of
             // a wavefront complete in order, so its next scan reads them
@@ -2200,8 +2156,6 @@ __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const S
                 } else if (lane == 7 && planner) {
                     // marks the move accepted: a decided move's particle index is not read again in this chunk
                     pk[m0 + k] |= PK_ACCEPTED;
-                } else if (G32 && lane >= 17 && lane < 20) {
-                    Sf[(lane - 17) * P.cap + ki] = reinterpret_cast<const float *>(q + 22)[lane - 17];
                 } else if (planner && lane >= 8 && lane < 17) {
                     oo[(lane - 8) * OWN_CAP + ki] = q[13 + (lane - 8)];
                 }
@@ -2211,8 +2165,8 @@ __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const S
                 // the next group was planned from a pose this group just replaced
                 __syncthreads();
                 if (planner)
-                    plan_group<KIND, TRANSLATED, G32 != 0>(P, S, oo, pt, pR, pk, sT, m1, gsNext, cell,
-                                                           plans + nbuf * GROUP * PLAN_D, plansI + nbuf * GPLAN_I, o);
+                    plan_group<KIND, TRANSLATED>(P, S, oo, pt, pR, pk, sT, m1, gsNext, cell,
+                                                  plans + nbuf * GROUP * PLAN_D, plansI + nbuf * GPLAN_I);
                 __syncthreads();
             }
             if (clk) {
@@ -2249,21 +2203,600 @@ __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const S
         P.p.wbits[gi] = (uint8_t)(((code & 3) - 1) | ((((code >> 2) & 3) - 1) << 1) | ((((code >> 4) & 3) - 1) << 2));
     }
     flush_counters(P, cell, accepted, moves, leftCell, tests, true);
-    if (G32 && !planner) {
-        // per-wavefront sums of the lanes' statistics, one atomic each
-        for (int off = WAVE / 2; off > 0; off >>= 1) {
-            g32Guard += __shfl_xor(g32Guard, off);
-            g32Mismatch += __shfl_xor(g32Mismatch, off);
-            g32Err = fmaxf(g32Err, __shfl_xor(g32Err, off));
-        }
-        if (lane == 0) {
-            if (wave == 1) P.slots[(size_t)cell * SLOT_WORDS + SLOT_G32_PAIRS] = g32Pairs;
-            if (g32Guard) atomicAdd(&P.counters[CNT_G32_GUARD], (unsigned long long)g32Guard);
-            if (G32 == 2) {
-                if (g32Mismatch) atomicAdd(&P.counters[CNT_G32_MISMATCH], (unsigned long long)g32Mismatch);
-                atomicMax(&P.counters[CNT_G32_MAXERR], (unsigned long long)__float_as_uint(g32Err));
+}
+
+// Speculative sweep of one staged cell: every move of a chunk (a lane each, at most SPEC_MOVES) is planned from the
+// poses the cell has when the chunk starts and tested against the whole stencil at once; the moves are then decided in
+// order by one wavefront.  With outside particles fixed for the colour pass, the only thing that can change a later
+// move's test is an accepted earlier move of the own cell, so each move keeps two results:
+//   hitOut   one bit: the trial pose overlaps a particle outside the cell (final whatever is decided before it);
+//   ownHit   64 bits: the own particles its trial pose overlaps, each in the pose that particle has now.
+// A move is rejected if it leaves the cell, if hitOut is set or if any ownHit bit is.  All moves before the first that is
+// not rejected are therefore decided by one ballot; that move is accepted, its particle's pose replaced, the particle's
+// bit of every later move's ownHit tested again against the new pose (a lane per move), and later moves of the same
+// particle, whose trial poses start from the new pose, are marked stale: they are planned and scanned again, all stale
+// moves of the chunk in one scan, when the first of them comes up.  The decisions, and so the trajectory, are those
+// of one move at a time.
+//
+// The scan's unit of work is 64 candidates (a lane each) against at most eight moves; units are dealt to the wavefronts.
+// Three stages, each on full wavefronts: the centre distances; on the pairs within the range (queued), a separating
+// direction that settles most of them; on those left (queued again), the exact segment test.  A move known to hit an
+// outside particle is not tested further.
+//
+// G32 = 1 (guarded FP32): the distance stage takes positions relative to the cell's centre in FP32 and keeps every pair
+// below the upper end of the guard band around range^2 (g32Lim), which is wider than the largest FP32 error the
+// positions' magnitudes allow; the later stages are FP64 and the same, so every decision equals the FP64 sweep's.
+// G32 = 2 also evaluates every pair in FP64 and records the largest FP32 error and any class that differs (none may).
+//
+// What bounds it: the arithmetic of the scan and its instruction issue (two workgroups, 16 wavefronts, per compute
+// unit); an accepted move costs about 1.2 us of one wavefront's latency.  Per workgroup on 1e5 rods (L/D 5, packing
+// fraction 0.45): staging 3.5 us, first scan 11.4, 1.2 rescans 2.8, 4.8 accepted moves 5.6; the groups of four moves
+// with a barrier each that this replaces took 52 us for the same moves.  100 cycles: 67.0 -> 51.5 ms on 1e5 rods,
+// 43.9 -> 38.6 ms on 8 000 (guarded), 50 cycles on 1e6: 414 -> 207 ms.
+constexpr int SPEC_MOVES = 32;     // moves per chunk
+constexpr int SPEC_PLAN = 19;      // doubles per plan: npos 3, NO 9, capA 3, u 3, a 1 (component c of move m at c * 32 + m)
+constexpr int SPEC_UNIT = 8;       // moves per unit of the first scan
+constexpr double SPEC_FAR = 1e17;  // position of a trial pose that is not to be tested (no pair comes within range)
+constexpr int SPEC_QNEAR = WAVE + SPEC_UNIT * WAVE;  // pairs within the range: drained to below 64 before every unit
+constexpr int SPEC_QSEG = 2 * WAVE;                   // pairs for the segment test: drained to below 64 after every drain
+constexpr int SPEC_QUEUE = SPEC_QNEAR + SPEC_QSEG;    // entries (candidate << 5 | move, 16 bits) per wavefront
+constexpr int SPEC_CAP = 2048;                        // candidates an entry can name
+constexpr int SPEC_INTS = SPEC_MOVES + 2 * SPEC_MOVES + 6;  // plan words, ownHit, hitOut, command, moved 2, spare 2
+
+struct SpecLds {
+    double *oo;         // 9 x OWN_CAP own orientations
+    double *box;        // dims 9, inv 9, shift 3
+    double *sT;         // translation table
+    double *prop;       // the chunk's proposals: translation 3, rotation 9 (component c of move m at c * 32 + m)
+    double *plan;       // SPEC_PLAN x SPEC_MOVES
+    int *word;          // per move: wrap bits | inside << 3 | particle << 8
+    unsigned *ownHit;   // two words per move
+    unsigned *hitOut;   // one bit per move
+    unsigned *cmd;      // the moves the next scan tests (none: the chunk is decided)
+    unsigned *moved;    // two words: own particles with a new pose
+    uint16_t *queue;    // SPEC_QUEUE per wavefront
+    float *Sf, *sTf, *planF;  // guarded FP32: stencil positions (3 x cap), translation table, trial positions (3 x 32)
+};
+
+size_t spec_lds_bytes(int kind, int cap, int waves, int g32) {
+    return stencil_lds_bytes(kind, cap) + sizeof(double) * (9 * OWN_CAP + 21 + 81 + (12 + SPEC_PLAN) * SPEC_MOVES) +
+           sizeof(int) * SPEC_INTS + sizeof(uint16_t) * (kind == 0 ? 0 : waves * SPEC_QUEUE) +
+           (g32 ? sizeof(float) * (3 * (size_t)cap + 81 + 3 * SPEC_MOVES) : 0);
+}
+
+template <int KIND, int WAVES>
+__device__ __forceinline__ SpecLds carve_spec(double *rest, int cap) {
+    SpecLds L;
+    L.oo = rest;
+    L.box = L.oo + 9 * OWN_CAP;
+    L.sT = L.box + 21;
+    L.prop = L.sT + 81;
+    L.plan = L.prop + 12 * SPEC_MOVES;
+    L.word = reinterpret_cast<int *>(L.plan + SPEC_PLAN * SPEC_MOVES);
+    L.ownHit = reinterpret_cast<unsigned *>(L.word + SPEC_MOVES);
+    L.hitOut = L.ownHit + 2 * SPEC_MOVES;
+    L.cmd = L.hitOut + 1;
+    L.moved = L.cmd + 1;
+    L.queue = reinterpret_cast<uint16_t *>(L.moved + 4);
+    L.Sf = reinterpret_cast<float *>(L.queue + (KIND == 0 ? 0 : WAVES * SPEC_QUEUE));
+    L.sTf = L.Sf + 3 * cap;
+    L.planF = L.sTf + 81;
+    return L;
+}
+
+// The constants of the scan's tests, read from the kernel argument once: a field of the argument is a scalar load and a
+// wait wherever it is used.
+struct SpecConsts {
+    double contact2, range2, halfLen, skip2;
+    float lim[4];
+    int cap;
+};
+
+// Statistics of the guarded FP32 scan, per lane (pairs: per wavefront).
+struct SpecStats {
+    unsigned guard = 0, mismatch = 0;
+    unsigned long long pairs = 0;
+    float err = 0.f;
+};
+
+// A mask in LDS that other wavefronts may be adding bits to, as a scalar.
+__device__ __forceinline__ unsigned lds_mask(const unsigned *w) {
+    return (unsigned)__builtin_amdgcn_readfirstlane(
+        (int)__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// The trial pose of this lane's move of own particle kIdx (record gi): the plan, and its word (wrap bits | inside << 3 |
+// particle << 8).  FIRST: the pose comes from the records, else from LDS.
+template <int KIND, int G32, bool FIRST>
+__device__ __forceinline__ int spec_plan(const SweepParams &P, const Stencil &S, const SpecLds &L, int lane, int kIdx,
+                                         int gi, int cell, const V3 &o) {
+    constexpr int M = SPEC_MOVES;
+    const Grid &g = P.g;
+    const double *pr = L.prop + lane;
+    double *q = L.plan + lane;
+    // the rotation a row at a time: few values live at once
+    V3 nax;
+    {
+        // Shape::rotate (Shape.cpp:14-16), the sums of mulm
+        double O[9];
+        for (int c = 0; c < 9; c++) O[c] = FIRST ? P.p.o[c][gi] : L.oo[c * OWN_CAP + kIdx];
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            const double r0 = pr[(3 + 3 * r) * M], r1 = pr[(4 + 3 * r) * M], r2 = pr[(5 + 3 * r) * M];
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                double v = 0;
+                v += r0 * O[c];
+                v += r1 * O[3 + c];
+                v += r2 * O[6 + c];
+                q[(3 + 3 * r + c) * M] = v;
+                if (c == 2) (r == 0 ? nax.x : r == 1 ? nax.y : nax.z) = v;
             }
         }
+    }
+    const V3 pos = FIRST ? load3(P.p.x, P.p.y, P.p.z, gi) : v3(S.x[kIdx], S.y[kIdx], S.z[kIdx]);
+    const V3 npos = translate_wrapped(L.box, L.box + 9, pos, v3(pr[0], pr[M], pr[2 * M]));
+    int nc[3];
+    unsigned nw;
+    bin_shifted(L.box + 9, L.box + 18, g.n, npos, nc, nw);
+    const int inside = cell_index(g, nc[0], nc[1], nc[2]) == cell ? 1 : 0;
+    q[0] = inside ? npos.x : SPEC_FAR;
+    q[M] = npos.y;
+    q[2 * M] = npos.z;
+    if (KIND == 1) {
+        const SCFirst f = sc_first(P.k, npos, nax);
+        q[12 * M] = f.capA.x;
+        q[13 * M] = f.capA.y;
+        q[14 * M] = f.capA.z;
+        q[15 * M] = f.u.x;
+        q[16 * M] = f.u.y;
+        q[17 * M] = f.u.z;
+        q[18 * M] = f.a;
+    }
+    if (G32) {
+        L.planF[lane] = inside ? (float)(npos.x - o.x) : (float)SPEC_FAR;
+        L.planF[M + lane] = (float)(npos.y - o.y);
+        L.planF[2 * M + lane] = (float)(npos.z - o.z);
+    }
+    // without the wrap bits of a move that leaves the cell, translation indices stay inside the 27-entry table
+    const int word = (inside ? (int)nw | 8 : 0) | (kIdx << 8);
+    L.word[lane] = word;
+    return word;
+}
+
+// Proposal i of the cycle into column `lane` of the chunk's proposals.
+__device__ __forceinline__ void spec_proposal(const SweepParams &P, const SpecLds &L, int lane, int i) {
+    for (int c = 0; c < 3; c++) L.prop[c * SPEC_MOVES + lane] = P.pr.t[c * P.pr.stride + i];
+    for (int c = 0; c < 9; c++) L.prop[(3 + c) * SPEC_MOVES + lane] = P.pr.R[c * P.pr.stride + i];
+}
+
+// Whether a pair of spherocylinders at centre difference d (axes a1, a2) certainly does not overlap.  For any direction
+// w the axis segments are at least (w.d - h |a1.w| - h |a2.w|) / |w| apart; with w the part of d across the first axis
+// this settles most pairs of a dense fluid's range sphere for a quarter of the segment test's operations.  skip2 is
+// the squared contact distance raised far beyond the rounding of these sums and of the exact test (SweepParams::skip2).
+__device__ __forceinline__ bool segments_apart(double halfLen, double skip2, const V3 &d, const V3 &a1, const V3 &a2) {
+    const V3 w = sub(d, scal(a1, dot(d, a1)));
+    const double t = dot(w, d) - halfLen * (fabs(dot(a1, w)) + fabs(dot(a2, w)));
+    return t > 0 && t * t > skip2 * dot(w, w);
+}
+
+__device__ __forceinline__ void spec_hit(const SpecLds &L, int j, int m, int nOwn) {
+    if (j < nOwn) atomicOr(&L.ownHit[2 * m + (j >> 5)], 1u << (j & 31));
+    else atomicOr(L.hitOut, 1u << m);
+}
+
+// The exact segment tests of at most 64 queued pairs, one per lane; pairs of moves already dead skip.
+__device__ __forceinline__ void spec_segments(const SpecConsts &K, const Stencil &S, const SpecLds &L, bool translated,
+                                              const uint16_t *entries, int n, int nOwn, unsigned dead) {
+    constexpr int M = SPEC_MOVES;
+    const int lane = threadIdx.x & (WAVE - 1);
+    __builtin_amdgcn_wave_barrier();  // the queue was written by other lanes of this wavefront
+    if (lane < n) {
+        const int e = entries[lane], j = e >> 5, m = e & (M - 1);
+        if (!((dead >> m) & 1)) {
+            V3 c2 = v3(S.x[j], S.y[j], S.z[j]);
+            if (!translated) {
+                const int w = L.word[m];
+                c2 = add(c2, image_translation(L.sT, S.code[j], w & 1, (w >> 1) & 1, (w >> 2) & 1));
+            }
+            const V3 a2 = v3(S.ax[j], S.ay[j], S.az[j]);
+            const double *p = L.plan + m;
+            const V3 c2a = add(c2, scal(a2, -K.halfLen));
+            const V3 c2b = add(c2, scal(a2, K.halfLen));
+            if (segment_distance2(v3(p[12 * M], p[13 * M], p[14 * M]), v3(p[15 * M], p[16 * M], p[17 * M]), p[18 * M],
+                                  c2a, c2b) < K.contact2)
+                spec_hit(L, j, m, nOwn);
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The near tests of at most 64 queued pairs, one per lane: in contact by the centre distance (a hit), beyond the range,
+// or separated (dropped), else queued for the segment test.  segQueued: entries of the second queue (updated).
+__device__ __forceinline__ void spec_near(const SpecConsts &K, const Stencil &S, const SpecLds &L, bool translated,
+                                          const uint16_t *entries, int n, uint16_t *segQueue, int &segQueued, int nOwn,
+                                          unsigned dead) {
+    constexpr int M = SPEC_MOVES;
+    const int lane = threadIdx.x & (WAVE - 1);
+    __builtin_amdgcn_wave_barrier();  // the queue was written by other lanes of this wavefront
+    bool keep = false;
+    int e = 0;
+    if (lane < n) {
+        e = entries[lane];
+        const int j = e >> 5, m = e & (M - 1);
+        if (!((dead >> m) & 1)) {
+            const int w = L.word[m];
+            V3 p2 = v3(S.x[j], S.y[j], S.z[j]);
+            if (!translated) p2 = add(p2, image_translation(L.sT, S.code[j], w & 1, (w >> 1) & 1, (w >> 2) & 1));
+            const double *p = L.plan + m;
+            const V3 d = sub(p2, v3(p[0], p[M], p[2 * M]));
+            const double d2 = dot(d, d);
+            if (j == (w >> 8)) {
+                // the moved particle itself
+            } else if (d2 < K.contact2) {
+                spec_hit(L, j, m, nOwn);
+            } else {
+                keep = d2 < K.range2 &&
+                       !segments_apart(K.halfLen, K.skip2, d, v3(p[5 * M], p[8 * M], p[11 * M]),
+                                       v3(S.ax[j], S.ay[j], S.az[j]));
+            }
+        }
+    }
+    const unsigned long long km = __ballot(keep);
+    if (keep)
+        segQueue[segQueued + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(km >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((unsigned)km, 0u))] = (uint16_t)e;
+    segQueued += __popcll(km);
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Squared centre distances of candidate p2 (fj: relative to the cell's centre, FP32) to NM trial poses, m[k] each, and
+// the pairs within the range queued; straight-line code, so that the moves' chains overlap.  A pose that is not to be
+// tested lies SPEC_FAR away.  The moved particle itself is queued as well; the near stage drops it.
+template <int NM, bool TRANSLATED, int G32>
+__device__ __forceinline__ void spec_unit(const SpecConsts &K, const SpecLds &L, const V3 &p2, const float *fj, int code,
+                                          int j, int nvalid, const int *m, uint16_t *nearQ, int &nearN, SpecStats &st) {
+    constexpr int M = SPEC_MOVES;
+    const int lane = threadIdx.x & (WAVE - 1);
+    double d2[NM];
+    float d2f[NM];
+    V3 q0 = p2;
+    if (!TRANSLATED && G32 != 1) q0 = add(p2, image_translation(L.sT, code, 0, 0, 0));
+#pragma unroll
+    for (int k = 0; k < NM; k++) {
+        int w = 0;
+        if (!TRANSLATED) w = __builtin_amdgcn_readfirstlane(L.word[m[k]]) & 7;
+        if (G32) {
+            float q[3] = {fj[0], fj[1], fj[2]};
+            if (!TRANSLATED) {
+                const int kx = (code & 3) - 1 - (w & 1), ky = ((code >> 2) & 3) - 1 - ((w >> 1) & 1),
+                          kz = ((code >> 4) & 3) - 1 - ((w >> 2) & 1);
+                const int t = 3 * ((kx + 1) * 9 + (ky + 1) * 3 + (kz + 1));
+                for (int c = 0; c < 3; c++) q[c] = q[c] + L.sTf[t + c];
+            }
+            const float dx = q[0] - L.planF[m[k]], dy = q[1] - L.planF[M + m[k]], dz = q[2] - L.planF[2 * M + m[k]];
+            d2f[k] = (dx * dx + dy * dy) + dz * dz;
+        }
+        if (G32 != 1) {
+            V3 q = q0;
+            if (!TRANSLATED && w) q = add(p2, image_translation(L.sT, code, w & 1, (w >> 1) & 1, (w >> 2) & 1));
+            const V3 d = sub(q, v3(L.plan[m[k]], L.plan[M + m[k]], L.plan[2 * M + m[k]]));
+            d2[k] = dot(d, d);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NM; k++) {
+        bool within;
+        if (G32) {
+            // the scan only has to keep every pair that may be in range: it compares with the upper end of the guard
+            // band, and the near stage classifies what it keeps from the FP64 distance
+            const float x = d2f[k];
+            within = x < K.lim[3];
+            if (within && ((x >= K.lim[0] && x < K.lim[1]) || x >= K.lim[2])) st.guard++;
+            if (G32 == 2 && lane < nvalid && d2[k] < 1e30) {
+                st.err = fmaxf(st.err, (float)fabs((double)x - d2[k]));
+                const bool c64 = d2[k] < K.contact2, w64 = d2[k] < K.range2;
+                if ((x < K.lim[0] && !c64) || (x >= K.lim[1] && c64) || (x < K.lim[2] && !w64) || (x >= K.lim[3] && w64))
+                    st.mismatch++;
+            }
+        } else {
+            within = d2[k] < K.range2;
+        }
+        const unsigned long long am = __ballot(within);
+        if (within)
+            nearQ[nearN + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(am >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo((unsigned)am, 0u))] =
+                (uint16_t)((j << 5) | m[k]);
+        nearN += __popcll(am);
+    }
+}
+
+// Scans the stencil for the moves of `active` (all inside the cell): the first scan of a chunk (whole = true: every
+// move that is not in `active` has its trial position SPEC_FAR away) in units of consecutive moves, a rescan in
+// units of up to four of its moves.
+template <int KIND, int WAVES, int G32>
+__device__ __forceinline__ void spec_scan(const SpecConsts &K, const Stencil &S, const SpecLds &L, bool translated,
+                                          int nOwn, int total, unsigned active, bool whole, SpecStats &st) {
+    static_assert(KIND == 1, "the queues serve spherocylinders");
+    constexpr int UNIT = G32 == 1 ? SPEC_UNIT : G32 == 0 ? SPEC_UNIT / 2 : 2;  // FP64 distances take more registers
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    uint16_t *nearQ = L.queue + wave * SPEC_QUEUE, *segQ = nearQ + SPEC_QNEAR;
+    int nearN = 0, segN = 0;
+    const int nslots = (total + WAVE - 1) / WAVE;
+    const unsigned skipDead = G32 == 2 ? 0u : ~0u;  // verify mode evaluates every pair
+    unsigned dead = lds_mask(L.hitOut) & skipDead;
+    int s = wave, grp = 0;
+    unsigned rest = active;  // rescans: the moves of this and the later groups
+    int ngroups = whole ? (SPEC_MOVES - __builtin_clz(active) + UNIT - 1) / UNIT : (__popc(active) + 3) / 4;
+    for (;;) {
+        while (s >= nslots) {
+            s -= nslots;
+            grp++;
+            if (!whole)
+                for (int k = 0; k < 4; k++) rest &= rest - 1;  // (stays 0 once it is)
+        }
+        if (grp >= ngroups) break;
+        const int j = s * WAVE + lane;
+        const bool valid = j < total;
+        const int jj = valid ? j : 0;
+        V3 p2;
+        float fj[3];
+        // lanes past the end hold a candidate nothing is near
+        if (G32 != 1) p2 = v3(valid ? S.x[jj] : -SPEC_FAR, S.y[jj], S.z[jj]);
+        if (G32) {
+            fj[0] = valid ? L.Sf[jj] : -1e17f;
+            fj[1] = L.Sf[K.cap + jj];
+            fj[2] = L.Sf[2 * K.cap + jj];
+        }
+        const int code = translated ? 0 : S.code[jj];
+        const int nvalid = min(WAVE, total - s * WAVE);
+        if (whole) {
+            const unsigned todo = (active >> (UNIT * grp)) & ((1u << UNIT) - 1);
+            if (todo & ~(dead >> (UNIT * grp))) {
+                int m[UNIT];
+                for (int k = 0; k < UNIT; k++) m[k] = UNIT * grp + k;
+                if (translated) spec_unit<UNIT, true, G32>(K, L, p2, fj, code, j, nvalid, m, nearQ, nearN, st);
+                else spec_unit<UNIT, false, G32>(K, L, p2, fj, code, j, nvalid, m, nearQ, nearN, st);
+                if (G32) st.pairs += (unsigned)(nvalid * __popc(todo));
+            }
+        } else {
+            // one unit per move (stale moves are few)
+            unsigned r = rest;
+            for (int k = 0; k < 4 && r; k++, r &= r - 1) {
+                const int m[1] = {__builtin_ctz(r)};
+                if (translated) spec_unit<1, true, G32>(K, L, p2, fj, code, j, nvalid, m, nearQ, nearN, st);
+                else spec_unit<1, false, G32>(K, L, p2, fj, code, j, nvalid, m, nearQ, nearN, st);
+                if (G32) st.pairs += (unsigned)nvalid;
+            }
+        }
+        while (nearN >= WAVE) {
+            nearN -= WAVE;
+            spec_near(K, S, L, translated, nearQ + nearN, WAVE, segQ, segN, nOwn, dead);
+            if (segN >= WAVE) {
+                segN -= WAVE;
+                spec_segments(K, S, L, translated, segQ + segN, WAVE, nOwn, dead);
+                dead |= lds_mask(L.hitOut) & skipDead;
+            }
+        }
+        s += WAVES;
+    }
+    if (nearN > 0) spec_near(K, S, L, translated, nearQ, nearN, segQ, segN, nOwn, dead);
+    while (segN > 0) {
+        const int n = min(segN, WAVE);
+        segN -= n;
+        spec_segments(K, S, L, translated, segQ + segN, n, nOwn, dead);
+    }
+}
+
+// The caller has planned the first chunk (its lanes' words in firstWord); total <= K.cap and nOwn <= OWN_CAP.
+template <int KIND, int WAVES, int G32>
+__device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, const Stencil &S, const SpecLds &L,
+                                                       bool translated, int own0, int nOwn, int total, int cell,
+                                                       int firstWord, unsigned long long *clk, const V3 &o) {
+    const int tid = threadIdx.x;
+    const int lane = tid & (WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    __shared__ unsigned long long sPairs;
+    const int moves = P.moves > 0 ? P.moves : nOwn * P.mult;
+    const int pbase = P.moves > 0 ? cell * P.moves : own0 * P.mult;
+    unsigned long long accepted = 0, leftCell = 0, tests = 0, moved = 0;
+    SpecStats st;
+    SpecConsts K;
+    K.contact2 = P.k.contact2;
+    K.range2 = P.k.range2;
+    K.halfLen = P.k.halfLen;
+    K.skip2 = P.skip2;
+    K.cap = P.cap;
+    if (G32)
+        for (int i = 0; i < 4; i++) K.lim[i] = P.g32Lim[translated ? 0 : 1][i];
+    unsigned long long tScan = 0, tRescan = 0, tDecide = 0, nRescans = 0;  // phase timers (clk)
+    if (G32 && tid == 0) sPairs = 0;
+    int word = firstWord;
+    for (int chunk = 0; chunk < moves; chunk += SPEC_MOVES) {
+        const int cn = min(SPEC_MOVES, moves - chunk);
+        if (wave == 0) {
+            if (chunk > 0 && lane < cn) {
+                spec_proposal(P, L, lane, pbase + chunk + lane);
+                word = spec_plan<KIND, G32, false>(P, S, L, lane, P.pr.k[pbase + chunk + lane], 0, cell, o);
+            }
+            const unsigned in = (unsigned)__ballot(lane < cn && (word & 8));
+            if (lane >= cn && lane < SPEC_MOVES) {
+                // the moves past the chunk's end
+                L.plan[lane] = SPEC_FAR;
+                L.plan[SPEC_MOVES + lane] = L.plan[2 * SPEC_MOVES + lane] = 0;
+                L.word[lane] = 0;
+                if (G32) {
+                    L.planF[lane] = (float)SPEC_FAR;
+                    L.planF[SPEC_MOVES + lane] = L.planF[2 * SPEC_MOVES + lane] = 0;
+                }
+            }
+            if (lane < SPEC_MOVES) {
+                L.ownHit[2 * lane] = 0;
+                L.ownHit[2 * lane + 1] = 0;
+            }
+            if (lane == 0) {
+                *L.hitOut = 0;
+                *L.cmd = in;
+            }
+        }
+        __syncthreads();  // the plans (and, for the first chunk, the staged stencil) are complete
+        int cur = 0;           // wavefront 0: the first undecided move,
+        unsigned accMask = 0;  // the accepted moves
+        for (int round = 0;; round++) {
+            const unsigned cmd = lds_mask(L.cmd);
+            if (!cmd) break;
+            const unsigned long long tc0 = clk ? wall_clock64() : 0;
+            spec_scan<KIND, WAVES, G32>(K, S, L, translated, nOwn, total, cmd, round == 0, st);
+            __syncthreads();  // every hit of this scan is in LDS
+            const unsigned long long tc1 = clk ? wall_clock64() : 0;
+            if (clk) {
+                tScan += round ? 0 : tc1 - tc0;
+                tRescan += round ? tc1 - tc0 : 0;
+                nRescans += round ? 1 : 0;
+            }
+            if (wave == 0) {
+                constexpr int M = SPEC_MOVES;
+                const int kIdx = word >> 8;
+                const int lm = lane & (M - 1);
+                unsigned mLo = L.ownHit[2 * lm], mHi = L.ownHit[2 * lm + 1];
+                unsigned out = lds_mask(L.hitOut);
+                bool stale = false;
+                unsigned next = 0;
+                const double *p = L.plan + lm;
+                V3 tp = v3(p[0], p[M], p[2 * M]), ta = v3(p[5 * M], p[8 * M], p[11 * M]);  // this lane's trial pose
+                for (;;) {
+                    const bool alive = lane < cn && (word & 8) && !((out >> lm) & 1);
+                    const unsigned staleMask = (unsigned)__ballot(stale);
+                    const unsigned ev = (unsigned)__ballot(lane >= cur && (stale || (alive && !(mLo | mHi))));
+                    if (!ev) break;
+                    const int a = __builtin_ctz(ev);
+                    if ((staleMask >> a) & 1) {
+                        // plan the stale moves from the current poses; scan again those that stay in the cell
+                        if (stale) {
+                            word = spec_plan<KIND, G32, false>(P, S, L, lane, kIdx, 0, cell, o);
+                            mLo = mHi = 0;
+                        }
+                        tp = v3(p[0], p[M], p[2 * M]);
+                        ta = v3(p[5 * M], p[8 * M], p[11 * M]);
+                        out &= ~staleMask;
+                        next = (unsigned)__ballot(stale && (word & 8));
+                        stale = false;
+                        cur = a;
+                        if (next) break;
+                        continue;
+                    }
+                    // accept move a (Packing::acceptMove: the cell belongs to this workgroup for the whole pass)
+                    const int wa = __builtin_amdgcn_readlane(word, a);
+                    const int ka = wa >> 8, na = wa & 7;
+                    accMask |= 1u << a;
+                    moved |= 1ull << ka;
+                    const double *q = L.plan + a;
+                    if (lane < (KIND == 1 ? 6 : 3)) {
+                        const int c = lane < 3 ? lane : 3 + 2 + 3 * (lane - 3);
+                        S.x[lane * K.cap + ka] = q[c * M];
+                    } else if (lane == 6) {
+                        S.code[ka] = wrap_code((unsigned)na);
+                    } else if (lane >= 8 && lane < 17) {
+                        L.oo[(lane - 8) * OWN_CAP + ka] = q[(3 + lane - 8) * M];
+                    } else if (G32 && lane >= 17 && lane < 20) {
+                        L.Sf[(lane - 17) * K.cap + ka] = L.planF[(lane - 17) * M + a];
+                    }
+                    // later moves: those of this particle are stale; the others meet its new pose
+                    const bool later = lane > a && lane < cn;
+                    if (later && kIdx == ka) stale = true;
+                    const bool test = later && kIdx != ka && alive && !stale;
+                    if (__any(test)) {
+                        V3 p2 = v3(q[0], q[M], q[2 * M]);
+                        if (!translated)
+                            p2 = add(p2, image_translation(L.sT, wrap_code((unsigned)na), word & 1, (word >> 1) & 1,
+                                                           (word >> 2) & 1));
+                        const V3 d = sub(p2, tp);
+                        const double d2 = dot(d, d);
+                        bool hit = test && d2 < K.contact2;
+                        if (KIND == 1) {
+                            const V3 a2 = v3(q[5 * M], q[8 * M], q[11 * M]);
+                            const bool close = test && !hit && d2 < K.range2 &&
+                                               !segments_apart(K.halfLen, K.skip2, d, ta, a2);
+                            if (__any(close)) {
+                                if (close) {
+                                    const V3 c2a = add(p2, scal(a2, -K.halfLen));
+                                    const V3 c2b = add(p2, scal(a2, K.halfLen));
+                                    hit = segment_distance2(v3(p[12 * M], p[13 * M], p[14 * M]),
+                                                            v3(p[15 * M], p[16 * M], p[17 * M]), p[18 * M], c2a,
+                                                            c2b) < K.contact2;
+                                }
+                            }
+                        }
+                        if (test) {
+                            const unsigned bit = 1u << (ka & 31);
+                            if (ka < 32) mLo = (mLo & ~bit) | (hit ? bit : 0u);
+                            else mHi = (mHi & ~bit) | (hit ? bit : 0u);
+                        }
+                    }
+                    cur = a + 1;
+                }
+                __builtin_amdgcn_wave_barrier();
+                if (next && lane < M) {
+                    // the scan ORs into these; the moves it does not test keep their results
+                    L.ownHit[2 * lane] = mLo;
+                    L.ownHit[2 * lane + 1] = mHi;
+                }
+                if (lane == 0) {
+                    *L.hitOut = out;
+                    *L.cmd = next;
+                }
+            }
+            if (clk) tDecide += wall_clock64() - tc1;
+            __syncthreads();  // the command, the plans and the poses of the next scan (or of the next chunk)
+        }
+        if (wave == 0) {
+            const int in = __popcll(__ballot(lane < cn && (word & 8)));
+            accepted += (unsigned long long)__popc(accMask);
+            leftCell += (unsigned long long)(cn - in);
+            tests += (unsigned long long)total * (unsigned long long)in;
+            if (P.pr.acc && lane < cn && ((accMask >> (lane & 31)) & 1)) P.pr.acc[pbase + chunk + lane] = 1;
+        }
+    }
+    if (wave == 0 && lane < 2) L.moved[lane] = (unsigned)(moved >> (32 * lane));
+    if (clk) {
+        clk[3] = wall_clock64();
+        if (tid == 0) {
+            atomicAdd(&P.phases[RP_PHASE_PLAN], tScan);
+            atomicAdd(&P.phases[RP_PHASE_SCAN], tRescan);
+            atomicAdd(&P.phases[RP_PHASE_DECIDE], tDecide);
+            atomicAdd(&P.phases[RP_PHASE_GROUPS], accepted);
+            atomicAdd(&P.phases[RP_PHASE_REPLANS], nRescans);
+        }
+    }
+    __syncthreads();
+    const unsigned long long changed = (unsigned long long)lds_mask(L.moved) | ((unsigned long long)lds_mask(L.moved + 1) << 32);
+    if (tid < nOwn && ((changed >> tid) & 1)) {
+        const int gi = own0 + tid;
+        P.p.x[gi] = S.x[tid];
+        P.p.y[gi] = S.y[tid];
+        P.p.z[gi] = S.z[tid];
+        for (int c = 0; c < 9; c++) P.p.o[c][gi] = L.oo[c * OWN_CAP + tid];
+        const int code = S.code[tid];
+        P.p.wbits[gi] = (uint8_t)(((code & 3) - 1) | ((((code >> 2) & 3) - 1) << 1) | ((((code >> 4) & 3) - 1) << 2));
+    }
+    flush_counters(P, cell, accepted, moves, leftCell, tests, true);
+    if (G32) {
+        for (int off = WAVE / 2; off > 0; off >>= 1) {
+            st.guard += __shfl_xor(st.guard, off);
+            st.mismatch += __shfl_xor(st.mismatch, off);
+            st.err = fmaxf(st.err, __shfl_xor(st.err, off));
+        }
+        if (lane == 0) {
+            atomicAdd(&sPairs, st.pairs);
+            if (st.guard) atomicAdd(&P.counters[CNT_G32_GUARD], (unsigned long long)st.guard);
+            if (G32 == 2) {
+                if (st.mismatch) atomicAdd(&P.counters[CNT_G32_MISMATCH], (unsigned long long)st.mismatch);
+                atomicMax(&P.counters[CNT_G32_MAXERR], (unsigned long long)__float_as_uint(st.err));
+            }
+        }
+        __syncthreads();
+        if (tid == 0) P.slots[(size_t)cell * SLOT_WORDS + SLOT_G32_PAIRS] = sPairs;
     }
 }
 
@@ -2462,8 +2995,8 @@ __device__ __forceinline__ void sweep_cell_soft(const SweepParams &P, const Sten
 template <int KIND, int NT, bool G32 = false>
 __device__ __forceinline__ void stage_stencil_batched(const SweepParams &P, const Stencil &S, const double *sT,
                                                       int total, bool translated, float *fx = nullptr,
-                                                      V3 o = V3{}) {
-    const int tid = threadIdx.x;
+                                                      V3 o = V3{}, int first = 0) {
+    const int tid = (int)threadIdx.x - first;  // NT threads from `first` on
     for (int base = 0; base < total; base += NT * SLOT_GROUP) {
         int gi[SLOT_GROUP], code[SLOT_GROUP];
 #pragma unroll
@@ -2511,6 +3044,15 @@ __device__ __forceinline__ void stage_stencil_batched(const SweepParams &P, cons
     }
 }
 
+__device__ __forceinline__ void trace_block(const SweepParams &P, int b, unsigned long long t0, int nOwn, int total,
+                                            int cell) {
+    unsigned long long *t = P.trace + 4 * b;
+    t[0] = t0;
+    t[1] = wall_clock64();
+    t[2] = (unsigned long long)nOwn | ((unsigned long long)total << 16) | ((unsigned long long)cell << 32);
+    t[3] = (unsigned long long)__smid();
+}
+
 // Active cell b of colour P.colour (one workgroup).
 // LEAN != 0: the kernel carries only the grouped sweep of staged cells (and the HBM path for cells that cannot be
 // staged), with fewer live registers than the general kernel: 1 FP64 scan, 2 guarded FP32 scan, 3 guarded FP32 scan
@@ -2554,6 +3096,66 @@ __device__ __forceinline__ void sweep_block(const SweepParams &P, const int b) {
     S.ncells = ncells;
     double *rest;
     carve_stencil(S, smem, P.cap, KIND, rest);
+    // with one cell across an axis the own cell recurs in its stencil under other images; staged copies would go
+    // stale as particles move, so such grids read the stencil from HBM
+    const bool ownRecurs = g.n[0] == 1 || g.n[1] == 1 || g.n[2] == 1;
+    if constexpr (LEAN != 0) {
+        const SpecLds L = carve_spec<KIND, WAVES>(rest, P.cap);
+        for (int i = tid; i < 81; i += NT) {
+            L.sT[i] = g.T[i];
+            if (G32) L.sTf[i] = (float)g.T[i];
+        }
+        if (tid < 21) L.box[tid] = tid < 9 ? g.dims[tid] : tid < 18 ? g.inv[tid - 9] : g.shift[tid - 18];
+        __syncthreads();
+        if (total <= P.cap && nOwn <= OWN_CAP && !ownRecurs) {
+            // a cell off the last row on every axis holds no wrapped particle: stage pos + T directly
+            const bool translated = cx < g.n[0] - 1 && cy < g.n[1] - 1 && cz < g.n[2] - 1;
+            // the guarded FP32 scan takes positions relative to the cell's centre
+            const V3 o = G32 ? mulv(g.dims, v3(g.shift[0] + ((double)cx + 0.5) * g.relCell[0],
+                                               g.shift[1] + ((double)cy + 0.5) * g.relCell[1],
+                                               g.shift[2] + ((double)cz + 0.5) * g.relCell[2]))
+                             : v3(0, 0, 0);
+            // the first wavefront plans the first moves from the global records while the others stage the stencil
+            int word = 0;
+            if (WAVES == 1 || tid < WAVE) {
+                const int moves = P.moves > 0 ? P.moves : nOwn * P.mult;
+                if (tid < min(SPEC_MOVES, moves)) {
+                    const int i = (P.moves > 0 ? cell * P.moves : own0 * P.mult) + tid, kIdx = P.pr.k[i];
+                    spec_proposal(P, L, tid, i);
+                    word = spec_plan<KIND, G32, true>(P, S, L, tid, kIdx, own0 + kIdx, cell, o);
+                }
+            }
+            constexpr int FIRST = WAVES == 1 ? 0 : WAVE;
+            if (tid >= FIRST) {
+                stage_stencil_batched<KIND, NT - FIRST, G32 != 0>(P, S, L.sT, total, translated, L.Sf, o, FIRST);
+                for (int e = tid - FIRST; e < 9 * nOwn; e += NT - FIRST) {
+                    const int c = e / nOwn, a = e - c * nOwn;
+                    L.oo[c * OWN_CAP + a] = P.p.o[c][own0 + a];
+                }
+            }
+            if (P.phases) clk[2] = wall_clock64();
+            unsigned long long *c3 = P.phases ? clk : nullptr;
+            sweep_cell_speculative<KIND, WAVES, G32>(P, S, L, translated, own0, nOwn, total, cell, word, c3, o);
+        } else {
+            if (P.phases) clk[2] = wall_clock64();
+            // proposals in the area of the chunk's proposals and plans
+            static_assert((12 + SPEC_PLAN) * SPEC_MOVES >= 12 * MOVE_CHUNK && 3 * SPEC_MOVES >= MOVE_CHUNK, "areas");
+            sweep_cell_unstaged<KIND, WAVES>(P, S, L.prop, L.prop + 3 * MOVE_CHUNK, L.word, L.sT, cell, own0, nOwn, total,
+                                             L.box, L.box + 9, L.box + 18);
+            if (P.phases) clk[3] = wall_clock64();
+        }
+        if (P.phases && tid == 0) {
+            clk[4] = wall_clock64();
+            atomicAdd(&P.phases[RP_PHASE_TABLE], clk[1] - clk[0]);
+            atomicAdd(&P.phases[RP_PHASE_STAGE], clk[2] - clk[1]);
+            atomicAdd(&P.phases[RP_PHASE_MOVES], clk[3] - clk[2]);
+            atomicAdd(&P.phases[RP_PHASE_WRITE], clk[4] - clk[3]);
+            atomicAdd(&P.phases[RP_PHASE_BLOCKS], 1ull);
+            atomicMax(&P.phases[RP_PHASE_LAST], clk[4] - clk[0]);
+        }
+        if (P.trace && tid == 0) trace_block(P, b, t0, nOwn, total, cell);
+        return;
+    }
     double *oo = rest;                  // 9 x OWN_CAP own orientations
     double *pt = oo + 9 * OWN_CAP;      // 3 x MOVE_CHUNK proposal translations
     double *pR = pt + 3 * MOVE_CHUNK;   // 9 x MOVE_CHUNK proposal rotations
@@ -2562,41 +3164,10 @@ __device__ __forceinline__ void sweep_block(const SweepParams &P, const int b) {
     int *pk = reinterpret_cast<int *>(plans + SWEEP_AUX);
     int *plansI = pk + MOVE_CHUNK;      // SWEEP_AUX_I planner output ints
     int *queue = plansI + SWEEP_AUX_I;  // max(cap + 64*WAVES, (WAVES-1)*GROUPED_QUEUE) queued candidates
-    // G32: the FP32 stencil positions (3 x cap) and translation table (81) after the queue
-    float *Sf = reinterpret_cast<float *>(queue + max(P.cap + WAVE * WAVES, (WAVES - 1) * GROUPED_QUEUE));
-    float *sTf = Sf + 3 * P.cap;
-    for (int i = tid; i < 81; i += NT) {
-        sT[i] = g.T[i];
-        if (G32) sTf[i] = (float)g.T[i];
-    }
+    for (int i = tid; i < 81; i += NT) sT[i] = g.T[i];
     __syncthreads();
 
-    // with one cell across an axis the own cell recurs in its stencil under other images; staged copies would go
-    // stale as particles move, so such grids read the stencil from HBM
-    const bool ownRecurs = g.n[0] == 1 || g.n[1] == 1 || g.n[2] == 1;
-    if (LEAN && KIND != 2 && total <= P.cap && nOwn <= OWN_CAP && !ownRecurs) {
-        // grouped moves only; the guarded FP32 scan takes positions relative to the cell's centre
-        const bool translated = cx < g.n[0] - 1 && cy < g.n[1] - 1 && cz < g.n[2] - 1;
-        const V3 o = G32 ? mulv(g.dims, v3(g.shift[0] + ((double)cx + 0.5) * g.relCell[0],
-                                           g.shift[1] + ((double)cy + 0.5) * g.relCell[1],
-                                           g.shift[2] + ((double)cz + 0.5) * g.relCell[2]))
-                         : v3(0, 0, 0);
-        stage_stencil_batched<KIND, NT, G32 != 0>(P, S, sT, total, translated, Sf, o);
-        for (int e = tid; e < 9 * nOwn; e += NT) {
-            int c = e / nOwn, a = e - c * nOwn;
-            oo[c * OWN_CAP + a] = P.p.o[c][own0 + a];
-        }
-        __syncthreads();
-        int *hitWords = plansI + GBUF * GPLAN_I;
-        if (translated)
-            sweep_cell_grouped<KIND, WAVES, true, G32>(P, S, oo, pt, pR, pk, queue, sT, plans, plansI, hitWords, own0,
-                                                       nOwn, total, cell, nullptr, Sf, sTf, o);
-        else
-            sweep_cell_grouped<KIND, WAVES, false, G32>(P, S, oo, pt, pR, pk, queue, sT, plans, plansI, hitWords, own0,
-                                                        nOwn, total, cell, nullptr, Sf, sTf, o);
-    } else if (LEAN) {
-        sweep_cell_unstaged<KIND, WAVES>(P, S, pt, pR, pk, sT, cell, own0, nOwn, total);
-    } else if (KIND != 2 && total <= P.cap && nOwn <= OWN_CAP && !ownRecurs) {
+    if (KIND != 2 && total <= P.cap && nOwn <= OWN_CAP && !ownRecurs) {
         // a cell off the last row on every axis holds no wrapped particle: stage pos + T directly
         const bool translated = cx < g.n[0] - 1 && cy < g.n[1] - 1 && cz < g.n[2] - 1;
         stage_stencil_batched<KIND, NT>(P, S, sT, total, translated);
@@ -2643,7 +3214,7 @@ __device__ __forceinline__ void sweep_block(const SweepParams &P, const int b) {
         if (SOFT)
             sweep_cell_soft<KIND, WAVES, false, false>(P, S, oo, pt, pR, pk, plans, sT, cell, own0, nOwn, total);
         else
-            sweep_cell_unstaged<KIND, WAVES>(P, S, pt, pR, pk, sT, cell, own0, nOwn, total);
+            sweep_cell_unstaged<KIND, WAVES>(P, S, pt, pR, pk, sT, cell, own0, nOwn, total, g.dims, g.inv, g.shift);
         if (P.phases) clk[3] = wall_clock64();
     }
     if (P.phases && tid == 0) {
@@ -2655,18 +3226,23 @@ __device__ __forceinline__ void sweep_block(const SweepParams &P, const int b) {
         atomicAdd(&P.phases[RP_PHASE_BLOCKS], 1ull);
         atomicMax(&P.phases[RP_PHASE_LAST], clk[4] - clk[0]);
     }
-    if (P.trace && tid == 0) {
-        unsigned long long *t = P.trace + 4 * b;
-        t[0] = t0;
-        t[1] = wall_clock64();
-        t[2] = (unsigned long long)nOwn | ((unsigned long long)total << 16) | ((unsigned long long)cell << 32);
-        t[3] = (unsigned long long)__smid();
-    }
+    if (P.trace && tid == 0) trace_block(P, b, t0, nOwn, total, cell);
 }
 
 // Two workgroups of eight wavefronts share a compute unit only within 128 registers per lane (4 wavefronts per SIMD)
 template <int KIND, int WAVES, bool SOFT, int LEAN = 0>
 __global__ __launch_bounds__(WAVE *WAVES, WAVES >= 8 ? 4 : 1) void k_sweep(SweepParams P) {
+#ifdef __HIP_DEVICE_COMPILE__
+    // The speculative kernel reads its argument through the kernel-argument segment's address (P is the first and only
+    // argument): loads of fields of a by-value argument are hoisted to the entry, and several hundred scalar registers
+    // of them spill; these stay where they are used.
+    if constexpr (LEAN != 0) {
+        typedef const __attribute__((address_space(4))) SweepParams ConstParams;
+        ConstParams *args = (ConstParams *)__builtin_amdgcn_kernarg_segment_ptr();
+        sweep_block<KIND, WAVES, SOFT, LEAN>(*(const SweepParams *)args, (int)blockIdx.x);
+        return;
+    }
+#endif
     sweep_block<KIND, WAVES, SOFT, LEAN>(P, (int)blockIdx.x);
 }
 
@@ -3156,6 +3732,12 @@ hipError_t launch_count_allpairs(hipStream_t s, const Grid &g, int n, Particles 
     return hipGetLastError();
 }
 
+int sweep_lean_cap() { return SPEC_CAP; }
+
+bool sweep_is_lean(const PairConsts &k, int waves, int pipelined, bool counting) {
+    return waves == 8 && pipelined == 2 && !k.soft && !counting && k.kind == 1;
+}
+
 int sweep_occupancy(int kind, int cap, int waves) {
     int w = waves >= 8 ? 8 : (waves >= 4 ? 4 : (waves == 2 ? 2 : 1));
     size_t lds = sweep_lds_bytes(kind, cap, w);
@@ -3208,9 +3790,8 @@ hipError_t launch_sweep(hipStream_t s, const SweepParams &sp, int waves, Timed t
     // the lean kernels run spherocylinders only: their first launch on spheres (eight wavefronts forced onto sparse
     // stencils) faulted the GPU and the cause is not found, so spheres keep the general kernel
     if (g32 && (w != 8 || sp.pipelined != 2 || sp.fixMode || sp.k.kind != 1)) return hipErrorInvalidValue;
-    size_t lds = sweep_lds_bytes(sp.k.kind, sp.cap, w, g32);
-    // the default hard launch (eight wavefronts, grouped moves) runs the lean kernels
-    const bool lean = w == 8 && sp.pipelined == 2 && !sp.fixMode && !sp.k.soft && !sp.counting && sp.k.kind == 1;
+    const bool lean = !sp.fixMode && sweep_is_lean(sp.k, w, sp.pipelined, sp.counting != 0);
+    size_t lds = sweep_lds_bytes(sp.k.kind, sp.cap, w, g32, lean);
     if (lean) {
 #define RP_SWEEP_L(L) \
     hipExtLaunchKernelGGL((k_sweep<1, 8, false, L>), dim3(blocks), dim3(WAVE * 8), (uint32_t)lds, s, t.start, t.stop, 0, sp)
@@ -3252,7 +3833,7 @@ hipError_t launch_sweep(hipStream_t s, const SweepParams &sp, int waves, Timed t
 int sweep_batch_key(const SweepParams &sp, int waves, int g32) {
     if (sp.k.soft || sp.counting || sp.fixMode || sp.k.kind == 2 || sp.trace || sp.g.allPairs) return -1;
     int w = waves >= 8 ? 8 : (waves >= 4 ? 4 : (waves == 2 ? 2 : 1));
-    const bool lean = w == 8 && sp.pipelined == 2 && sp.k.kind == 1;  // as launch_sweep chooses
+    const bool lean = sweep_is_lean(sp.k, w, sp.pipelined, false);
     if (g32 && !lean) return -1;
     return sp.k.kind | (w << 4) | ((lean ? 1 + g32 : 0) << 8);
 }
