@@ -135,7 +135,7 @@ struct rp_ctx {
     bool sortedForCycle = false;
 
     // polyspheres: bead table on the device, total range, bead items for overlap counts
-    double *dBeads = nullptr;
+    double *dBeads = nullptr, *dGroups = nullptr;
     double totalRange = 0;
     double beadVolume = 0;  // sum of bead volumes (NaN when beads overlap)
     int *beadCellStart = nullptr, *beadCellCount = nullptr;  // cell arrays of bead grids (kept apart from the
@@ -348,6 +348,71 @@ int uploadBeads(const rp_shape_desc &s, double **dBeads) {
         *dBeads = nullptr;
         return fail(RP_ERR_DEVICE, "bead upload failed");
     }
+    return RP_OK;
+}
+
+// The bead groups and the capsule of the polysphere sweep: the long axis joins the two beads furthest apart, the beads
+// are sorted along it and split into at most four groups of equal size (the last may be smaller).  Radii are raised by a
+// relative 1e-12, beyond the rounding of their square roots.
+int uploadGroups(const rp_shape_desc &s, PairConsts &k, double **dGroups) {
+    *dGroups = nullptr;
+    if (s.kind != RP_SHAPE_POLYSPHERE) return RP_OK;
+    const int nc = s.n_centres;
+    auto at = [&](int i) { return v3(s.centres[3 * i], s.centres[3 * i + 1], s.centres[3 * i + 2]); };
+    V3 axis = v3(1, 0, 0);
+    double far2 = 0;
+    for (int i = 0; i < nc; i++)
+        for (int j = i + 1; j < nc; j++) {
+            const V3 d = sub(at(j), at(i));
+            if (dot(d, d) > far2) {
+                far2 = dot(d, d);
+                axis = scal(d, 1 / std::sqrt(far2));
+            }
+        }
+    k.capAxis[0] = axis.x;
+    k.capAxis[1] = axis.y;
+    k.capAxis[2] = axis.z;
+    k.capHalf = k.capRadius = 0;
+    std::vector<int> order(nc);
+    for (int i = 0; i < nc; i++) {
+        order[i] = i;
+        const double along = dot(at(i), axis);
+        const V3 across = sub(at(i), scal(axis, along));
+        k.capHalf = std::max(k.capHalf, std::fabs(along));
+        k.capRadius = std::max(k.capRadius, (std::sqrt(dot(across, across)) + s.radii[i]) * (1 + 1e-12));
+    }
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int i, int j) { return dot(at(i), axis) < dot(at(j), axis); });
+    k.groupSize = (nc + 3) / 4;
+    // four slots per group (a short group repeats its last bead), then the groups' bounding spheres
+    constexpr int groups = 4, slots = RP_MAX_CENTRES / groups;
+    std::vector<double> h(4 * (size_t)(RP_MAX_CENTRES + groups), 0.0);
+    for (int g = 0; g * k.groupSize < nc; g++) {
+        const int lo = g * k.groupSize, hi = std::min(nc, lo + k.groupSize);
+        V3 centre = v3(0, 0, 0);
+        for (int i = lo; i < hi; i++) centre = add(centre, scal(at(order[i]), 1.0 / (hi - lo)));
+        double radius = 0;
+        for (int slot = 0; slot < slots; slot++) {
+            const int i = order[std::min(lo + slot, hi - 1)];
+            const V3 d = sub(at(i), centre);
+            radius = std::max(radius, (std::sqrt(dot(d, d)) + s.radii[i]) * (1 + 1e-12));
+            double *q = &h[4 * (size_t)(g * slots + slot)];
+            for (int c = 0; c < 3; c++) q[c] = s.centres[3 * i + c];
+            q[3] = s.radii[i];
+        }
+        double *q = &h[4 * (size_t)(RP_MAX_CENTRES + g)];
+        q[0] = centre.x;
+        q[1] = centre.y;
+        q[2] = centre.z;
+        q[3] = radius;
+    }
+    RP_HIP(hipMalloc(dGroups, sizeof(double) * h.size()));
+    if (hipMemcpy(*dGroups, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice) != hipSuccess) {
+        hipFree(*dGroups);
+        *dGroups = nullptr;
+        return fail(RP_ERR_DEVICE, "bead upload failed");
+    }
+    k.groups = *dGroups;
     return RP_OK;
 }
 
@@ -1087,18 +1152,19 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
     int waves = c->sweepWaves;
     // eight wavefronts with grouped moves for dense stencils (measured fastest on 1e5 rods), else fewer
     if (waves <= 0) waves = expect > 384 ? 8 : (expect > 128 ? 2 : 1);
-    // polyspheres whose stencils hold over a thousand particles: sixteen (2.24e6 against 2.09e6 trial moves/s with
-    // eight on 50 653 kinked chains)
-    if (c->sweepWaves <= 0 && c->k.kind == RP_SHAPE_POLYSPHERE && expect > 1024) waves = 16;
+    // hard polyspheres: the speculative sweep on eight or sixteen wavefronts once a stencil holds some 200 particles, one
+    // move at a time below that (10 cycles on 5-bead chains, stencils of 270: 14.8 ms against 17.2 with two wavefronts one
+    // at a time; 3-bead chains, 130: 9.2 on four wavefronts against 7.7; 7-bead chains, 650: sixteen 16.0, eight 16.3)
+    if (c->sweepWaves <= 0 && c->k.kind == RP_SHAPE_POLYSPHERE && !c->counting)
+        waves = expect > 512 ? 16 : (expect > 192 ? 8 : (expect > 128 ? 2 : 1));
     waves = waves >= 16 ? 16 : (waves >= 8 ? 8 : (waves >= 4 ? 4 : (waves == 2 ? 2 : 1)));
-    // sixteen wavefronts only for the hard polysphere sweep (moves that scan thousands of stencil entries from HBM)
+    // sixteen wavefronts only for the hard polysphere sweep
     if (waves == 16 && (c->k.kind != RP_SHAPE_POLYSPHERE || c->k.soft || c->counting)) waves = 8;
-    // eight wavefronts only for the hard sweeps (polyspheres: 1.5x faster than four on 50 653 kinked chains, whose
-    // moves scan up to 2 350 stencil entries from HBM)
+    // eight wavefronts only for the hard sweeps
     if (waves == 8 && (c->k.soft || c->counting)) waves = 4;
     // per-sampler acceptance flags are compiled into the kernels of at most four wavefronts only (the eight-wavefront
     // kernel has no registers to spare for them)
-    if (waves >= 8 && ms.n > 1) waves = 4;
+    if (waves >= 8 && ms.n > 1 && c->k.kind != RP_SHAPE_POLYSPHERE) waves = 4;
     sp.pipelined = c->pipelined >= 0 ? c->pipelined : (waves >= 8 ? 2 : 1);
     // guarded FP32 stencil scan: the default launch of hard spherocylinders (eight wavefronts, grouped moves); the
     // all-pairs path (no grid) tests in FP64
@@ -1110,19 +1176,21 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
         // that of the sums it propagates through, is below 1e-13 of the extent
         double extent = 0;
         for (int i = 0; i < 9; i++) extent += std::fabs(g.dims[i]);
-        const double d = std::sqrt(c->k.contact2) * (1 + 1e-7) + 1e-11 * extent;
+        const double contact = c->k.kind == RP_SHAPE_POLYSPHERE ? 2 * c->k.capRadius : std::sqrt(c->k.contact2);
+        const double d = contact * (1 + 1e-7) + 1e-11 * extent;
         sp.skip2 = d * d;
     }
     const bool lean = sweep_is_lean(c->k, waves, sp.pipelined, c->counting && !c->k.soft);
+    const bool poly = c->k.kind == RP_SHAPE_POLYSPHERE;  // reads its stencil from HBM: no stencil area to size
     const size_t fixed = sweep_lds_bytes(c->k.kind, 0, waves, g32, lean);
     const double perEntry = (double)(sweep_lds_bytes(c->k.kind, 1024, waves, g32, lean) - fixed) / 1024.0;
-    int maxCap = (int)((double)(c->ldsLimit - fixed) / perEntry) / 64 * 64;
+    const int maxCap = poly ? 64 : (int)((double)(c->ldsLimit - fixed) / perEntry) / 64 * 64;
     sp.cap = std::max(64, std::min(cap, maxCap));
     if (lean) sp.cap = std::min(sp.cap, sweep_lean_cap());
     // workgroups that read their stencil from HBM so far (hCounters as of the last read)
     if (!c->pairCapOff && c->blocksAtRead >= 10000 && c->hCounters[CNT_UNSTAGED_BLOCKS] * 100 > c->blocksAtRead)
         c->pairCapOff = true;
-    if (waves == 8 && !c->pairCapOff) {
+    if (waves == 8 && !c->pairCapOff && !poly) {
         // two eight-wavefront workgroups share a compute unit (128 registers each) only if each takes at most half the
         // unit's LDS (ldsLimit is the unit's LDS less 4 KB; the kernel's static arrays take under 2 KB): a smaller
         // stencil area is worth it while it still holds the expected stencil with a margin of 3 standard deviations
@@ -1132,7 +1200,6 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
         const int pairCap = (int)((half - (double)fixed) / perEntry) / 64 * 64;
         if (pairCap < sp.cap && pairCap >= expect + 3 * std::sqrt(expect)) sp.cap = pairCap;
     }
-    if (c->k.kind == RP_SHAPE_POLYSPHERE) sp.cap = 64;  // the polysphere sweep reads its stencil from HBM
     if (g.allPairs) sp.cap = allPairsStaged(c);
     r = ensureSlots(c, g.ncell);
     if (r) return r;
@@ -1675,6 +1742,8 @@ int rp_create(rp_ctx **out, const rp_shape_desc *shape, const double box[9], siz
     if (hipStreamCreate(&c->stream) != hipSuccess) return cleanup(fail(RP_ERR_DEVICE, "hipStreamCreate failed"));
     int r = uploadBeads(*shape, &c->dBeads);
     if (r) return cleanup(r);
+    r = uploadGroups(*shape, c->k, &c->dGroups);
+    if (r) return cleanup(r);
     c->k.beads = c->dBeads;
     c->k.nc = shape->kind == RP_SHAPE_POLYSPHERE ? shape->n_centres : 0;
     // polysphere sweep prefilter: particles whose centres are at least the total range apart share no bead
@@ -2160,6 +2229,7 @@ void rp_destroy(rp_ctx *c) {
     if (c->beadA.mem) hipFree(c->beadA.mem);
     if (c->beadB.mem) hipFree(c->beadB.mem);
     if (c->dBeads) hipFree(c->dBeads);
+    if (c->dGroups) hipFree(c->dGroups);
     if (c->beadCellStart) hipFree(c->beadCellStart);
     if (c->beadCellCount) hipFree(c->beadCellCount);
     if (c->cellStart) hipFree(c->cellStart);

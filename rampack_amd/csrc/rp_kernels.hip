@@ -1295,8 +1295,10 @@ hipError_t launch_type_counts(hipStream_t s, const Proposals &pr, size_t total, 
 // lean: the speculative sweep's own layout (spec_lds_bytes).
 size_t spec_lds_bytes(int kind, int cap, int waves, int g32);
 
+size_t poly_lds_bytes(int waves);
+
 size_t sweep_lds_bytes(int kind, int cap, int waves, int g32, bool lean) {
-    if (lean) return spec_lds_bytes(kind, cap, waves, g32);
+    if (lean) return kind == 2 ? poly_lds_bytes(waves) : spec_lds_bytes(kind, cap, waves, g32);
     const int queueInts = max(cap + WAVE * waves, (waves - 1) * GROUPED_QUEUE);
     return stencil_lds_bytes(kind, cap) + sizeof(int) * queueInts +
            sizeof(double) * (9 * OWN_CAP + 12 * MOVE_CHUNK + 81 + SWEEP_AUX) + sizeof(int) * (MOVE_CHUNK + SWEEP_AUX_I);
@@ -2800,6 +2802,535 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
     }
 }
 
+// Speculative sweep of one polysphere cell: the scheme of sweep_cell_speculative (every move of a chunk tested at once,
+// then decided in order), for stencils of thousands of particles read from the cell-sorted records in HBM.
+//
+// The scan deals units of 64 stencil entries (a lane each) to the wavefronts, first those of the own cell and its
+// neighbours for all moves, then the others for the moves that overlap nothing so far.  A unit's records are loaded once
+// for several batches of four moves, each tested by the centre distance and -- if any lane is within range -- by a
+// separating direction of the capsules that hold the particles' beads.  The pairs left are queued, spread evenly over the
+// wavefronts, and take a lane per bead of the candidate: the lane compares its bead with the bounding spheres of the moved
+// particle's bead groups (at most four) and tests the beads of the groups within reach exactly.  Every filter keeps each
+// pair whose rounded bead test could be positive.
+//
+// Trial poses of the chunk's moves are tested against each other in the same scan (bit a of tt[m]: move m's trial pose
+// overlaps move a's), so accepting a move costs no further pair test: it copies one bit per later move.  A move that only
+// own particles stop is not scanned beyond the near cells until an accepted move frees it.
+//
+// What bounds it: the latency of the rounds; a colour pass has one workgroup per active cell, fewer than the chip has
+// compute units on 5e4 chains.  50 653 kinked 11-bead chains at p* 3, 8 cycles: 117 -> 31 ms; per workgroup (36 moves,
+// 2 800 entries) 55 us, of which the first scan 39, rescans 6.6, decisions 2.4.  Measured slower: a wavefront testing its
+// own queue (59 us for the first scan: the pairs of a layer crowd into a few units), and four or eight workgroups per
+// cell that share the first scan and hand over through atomics (the last one's records come cold: 36 ms).
+constexpr int POLY_MOVES = 64;                      // moves per chunk, a lane each
+constexpr int POLY_GROUPS = 4;                     // bead groups per particle, at most
+constexpr int POLY_BATCH = 4;                      // moves tested together
+constexpr int POLY_QUEUE = 640;                    // pairs queued per wavefront, at most
+constexpr int POLY_SLOTS = RP_MAX_CENTRES / POLY_GROUPS;  // beads per group, at most; a short group repeats its last bead
+constexpr int POLY_PLAN = 12 + 3 + 3 * RP_MAX_CENTRES + 3 * POLY_GROUPS;  // doubles per move: npos 3, NO 9, axis 3, trial
+                                                                         // bead centres, group centres
+constexpr int POLY_CONSTS = 81 + 21 + 4 * RP_MAX_CENTRES + 4 * POLY_GROUPS;
+static_assert(POLY_GROUPS * POLY_SLOTS == RP_MAX_CENTRES, "bead slots");
+// words of a chunk's results: ownHit 2 per move, tt 2 per move, hitOut 2; then scan 2, undecided 2, more 2, queue
+// lengths, plan words
+constexpr int POLY_RESULTS = 4 * POLY_MOVES + 2;
+constexpr int POLY_INTS = POLY_RESULTS + 6 + 16 + POLY_MOVES;
+
+struct PolyLds {
+    double *sT, *box;      // translation table; dims 9, inv 9, shift 3
+    double *beads;         // body-frame beads in group order: x, y, z, radius
+    double *group;         // bounding sphere of each group: x, y, z, radius
+    double *plan;          // POLY_PLAN x POLY_MOVES (component c of move m at c * 64 + m)
+    int *word;             // per move: wrap bits | inside << 3 | particle << 8
+    unsigned *ownHit;      // two words per move: own particles its trial pose overlaps
+    unsigned *tt;          // two words per move: earlier moves whose trial pose it overlaps
+    unsigned *hitOut;      // two words: a bit per move that overlaps an outside particle
+    unsigned *scan;        // two words: the moves the next scan tests
+    unsigned *undecided;   // two words: the moves whose trial poses it tests them against
+    unsigned *more;        // two words: stale moves (another round follows)
+    int *queued;           // pairs in each wavefront's queue
+    int *queue;            // per wavefront: POLY_QUEUE records (own trial pose a: -1 - a), POLY_QUEUE image code << 6 | move
+};
+
+size_t poly_lds_bytes(int waves) {
+    const size_t doubles = POLY_CONSTS + (size_t)POLY_PLAN * POLY_MOVES;
+    return sizeof(double) * doubles + sizeof(int) * (POLY_INTS + (size_t)waves * 2 * POLY_QUEUE);
+}
+
+__device__ __forceinline__ PolyLds carve_poly(double *smem) {
+    PolyLds L;
+    L.sT = smem;
+    L.box = L.sT + 81;
+    L.beads = L.box + 21;
+    L.group = L.beads + 4 * RP_MAX_CENTRES;
+    L.plan = L.group + 4 * POLY_GROUPS;
+    L.ownHit = reinterpret_cast<unsigned *>(L.plan + POLY_PLAN * POLY_MOVES);
+    L.tt = L.ownHit + 2 * POLY_MOVES;
+    L.hitOut = L.tt + 2 * POLY_MOVES;
+    L.scan = L.hitOut + 2;
+    L.undecided = L.scan + 2;
+    L.more = L.undecided + 2;
+    L.queued = reinterpret_cast<int *>(L.more + 2);
+    L.word = L.queued + 16;
+    L.queue = L.word + POLY_MOVES;
+    return L;
+}
+
+__device__ __forceinline__ unsigned long long lds_mask2(const unsigned *w) {
+    return (unsigned long long)lds_mask(w) | ((unsigned long long)lds_mask(w + 1) << 32);
+}
+
+struct PolyConsts {
+    double range2, skip2, halfLen;
+    V3 axis;
+    int groupSize, groups;
+    int pairShift, pairs;  // queued pairs tested together: sixteen of up to four beads, else four
+};
+
+// Whether two particles at centre difference d (capsule axes a1, a2) certainly share no bead contact: the capsules'
+// axis segments are further apart than twice their radius (skip2: that distance squared, raised beyond rounding).  w is
+// the part of d across the first axis, as in segments_apart; a1 has unit length up to rounding, so a1.w is nothing.
+__device__ __forceinline__ bool capsules_apart(double halfLen, double skip2, const V3 &d, const V3 &a1, const V3 &a2) {
+    const double s = fma(d.z, a1.z, fma(d.y, a1.y, d.x * a1.x));
+    const V3 w = v3(fma(-s, a1.x, d.x), fma(-s, a1.y, d.y), fma(-s, a1.z, d.z));
+    const double ww = fma(w.z, w.z, fma(w.y, w.y, w.x * w.x));
+    const double aw = fma(w.z, a2.z, fma(w.y, a2.y, w.x * a2.x));
+    const double t = fma(-halfLen, fabs(aw), ww);
+    return t > 0 && t * t > skip2 * ww;
+}
+
+// The exact tests of at most K.pairs queued pairs (entry: the lane's, or none), 64 / K.pairs lanes each: a lane has one of the candidate's beads and
+// tests it against the moved particle's bead groups whose bounding sphere it reaches (a relative 1e-9 covers the
+// rounding).  The lanes of a pair read the same moved beads, which the LDS broadcasts.  Pairs of dead moves skip.
+__device__ __forceinline__ void poly_pairs(const SweepParams &P, const PolyConsts &K, const PolyLds &L, const int *entry,
+                                           int own0, int nOwn) {
+    constexpr int M = POLY_MOVES;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const unsigned long long dead = lds_mask2(L.hitOut);
+    const int i = lane & ((1 << K.pairShift) - 1);
+    const int b = K.pairShift == 2 ? i * POLY_SLOTS : i;  // bead slot
+    if (entry && b / POLY_SLOTS < K.groups && b % POLY_SLOTS < K.groupSize) {
+        const int gj = entry[0], cm = entry[POLY_QUEUE], m = cm & (M - 1), code = cm >> 6;
+        if (gj < 0 || !((dead >> m) & 1)) {
+            const V3 bead = v3(L.beads[4 * b], L.beads[4 * b + 1], L.beads[4 * b + 2]);
+            const double rb = L.beads[4 * b + 3];
+            V3 c2;
+            {
+                double O[9];
+                V3 p2;
+                if (gj < 0) {
+                    const double *q = L.plan + (-1 - gj);
+                    p2 = v3(q[0], q[M], q[2 * M]);
+                    for (int c = 0; c < 9; c++) O[c] = q[(3 + c) * M];
+                } else {
+                    p2 = load3(P.p.x, P.p.y, P.p.z, gj);
+                    for (int c = 0; c < 9; c++) O[c] = P.p.o[c][gj];
+                }
+                c2 = add(p2, mulv(O, bead));
+            }
+            const int w = L.word[m];
+            const V3 T = image_translation(L.sT, code, w & 1, (w >> 1) & 1, (w >> 2) & 1);
+            const double *trial = L.plan + 15 * M + m, *centre = L.plan + (15 + 3 * RP_MAX_CENTRES) * M + m;
+            const V3 q2 = add(c2, T);
+            bool hit = false;
+#pragma unroll 1
+            for (int ga = 0; ga < K.groups; ga++) {
+                const V3 f = sub(q2, v3(centre[3 * ga * M], centre[(3 * ga + 1) * M], centre[(3 * ga + 2) * M]));
+                const double t = L.group[4 * ga + 3] + rb;
+                if (!(dot(f, f) > (t * t) * (1 + 1e-9))) {
+                    const double *q = trial + 3 * POLY_SLOTS * ga * M, *ra = L.beads + 4 * POLY_SLOTS * ga + 3;
+#pragma unroll
+                    for (int a = 0; a < POLY_SLOTS; a++)
+                        hit |= bead_overlap(ra[4 * a], rb, v3(q[3 * a * M], q[(3 * a + 1) * M], q[(3 * a + 2) * M]), c2, T);
+                }
+            }
+            if (hit) {
+                // bit `bit` of a two-word mask
+                unsigned *mask = L.hitOut;
+                int bit = m;
+                if (gj < 0) {
+                    mask = L.tt + 2 * m;
+                    bit = -1 - gj;
+                } else if (gj >= own0 && gj < own0 + nOwn) {
+                    mask = L.ownHit + 2 * m;
+                    bit = gj - own0;
+                }
+                atomicOr(mask + (bit >> 5), 1u << (bit & 31));
+            }
+        }
+    }
+}
+
+// Queues this lane's pair (if keep) and returns the queue's new length.
+__device__ __forceinline__ int poly_queue(bool keep, int gj, int cm, int *queue, int queued) {
+    const unsigned long long mask = __ballot(keep);
+    if (keep) {
+        const int at = queued + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+        queue[at] = gj;
+        queue[POLY_QUEUE + at] = cm;
+    }
+    return queued + __popcll(mask);
+}
+
+// Tests the last pairs of this wavefront's queue until a batch fits in it again (rarely needed).
+__device__ __forceinline__ int poly_make_room(const SweepParams &P, const PolyConsts &K, const PolyLds &L, const int *queue,
+                                              int queued, int own0, int nOwn) {
+    const int e = (int)(threadIdx.x & (WAVE - 1)) >> K.pairShift;
+    while (queued > POLY_QUEUE - POLY_BATCH * WAVE) {
+        queued -= K.pairs;
+        __builtin_amdgcn_wave_barrier();  // the queue was written by other lanes of this wavefront
+        poly_pairs(P, K, L, queue + queued + e, own0, nOwn);
+        __builtin_amdgcn_wave_barrier();
+    }
+    return queued;
+}
+
+// Tests the pairs of every wavefront's queue, spread evenly: the pairs of a layer crowd into a few units.
+template <int WAVES>
+__device__ __forceinline__ void poly_drain(const SweepParams &P, const PolyConsts &K, const PolyLds &L, int own0, int nOwn) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    const int end = wave_inclusive_scan(lane < WAVES ? L.queued[lane] : 0);
+    const int total = __builtin_amdgcn_readlane(end, WAVE - 1);
+    for (int base = wave * K.pairs; base < total; base += WAVES * K.pairs) {
+        const int e = base + (lane >> K.pairShift);
+        int w = 0, before = 0;
+#pragma unroll
+        for (int k = 0; k < WAVES; k++) {
+            const int stop = __builtin_amdgcn_readlane(end, k);
+            w += e >= stop ? 1 : 0;
+            before = e >= stop ? stop : before;
+        }
+        poly_pairs(P, K, L, e < total ? L.queue + w * 2 * POLY_QUEUE + (e - before) : nullptr, own0, nOwn);
+    }
+}
+
+// Stencil entries [unit0, unit1) x 64 against the moves of `active` in items of one unit and POLY_BATCH moves; this
+// wavefront has share `worker` of `workers`.  Returns the pairs left in its queue.
+__device__ __forceinline__ int poly_units(const SweepParams &P, const PolyConsts &K, const Stencil &S, const PolyLds &L,
+                                          int own0, int nOwn, int total, int unit0, int unit1, unsigned long long active,
+                                          int worker, int workers, int *queue, int queued) {
+    constexpr int M = POLY_MOVES;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int batches = (__popcll(active) + POLY_BATCH - 1) / POLY_BATCH;
+    int loaded = -1, gj = 0, j = 0, code = 0;
+    bool valid = false, haveAxis = false;
+    V3 a2, q0;
+    // consecutive items share a unit, whose records are then kept
+    const int items = (unit1 - unit0) * batches, first = items * worker / workers,
+              last = items * (worker + 1) / workers;
+    for (int item = first; item < last; item++) {
+        const int unit = unit0 + item / batches, batch = item % batches;
+        unsigned long long rest = active;
+        for (int k = 0; k < batch * POLY_BATCH; k++) rest &= rest - 1;
+        const unsigned long long dead = lds_mask2(L.hitOut);
+        int m[POLY_BATCH], w[POLY_BATCH];
+        unsigned use = 0;
+#pragma unroll
+        for (int k = 0; k < POLY_BATCH; k++) {
+            m[k] = rest ? __builtin_ctzll(rest) : m[0];
+            use |= rest && !((dead >> m[k]) & 1) ? 1u << k : 0u;
+            rest &= rest - 1;  // (0 stays 0)
+        }
+        if (!use) continue;
+        if (unit != loaded) {
+            loaded = unit;
+            j = unit * WAVE + lane;
+            valid = j < total;
+            const int jj = valid ? j : 0;
+            const int q = stencil_cell(S.start, S.ncells, jj);
+            gj = S.base[q] + (jj - S.start[q]);
+            const V3 p2 = load3(P.p.x, P.p.y, P.p.z, gj);
+            haveAxis = false;
+            code = image_code(S.ecode[q], P.p.wbits[gj]);
+            q0 = add(p2, image_translation(L.sT, code, 0, 0, 0));
+        }
+        bool in[POLY_BATCH], any = false;
+        V3 d[POLY_BATCH];
+#pragma unroll
+        for (int k = 0; k < POLY_BATCH; k++) w[k] = __builtin_amdgcn_readfirstlane(L.word[m[k]]);
+#pragma unroll
+        for (int k = 0; k < POLY_BATCH; k++) {
+            V3 q2 = q0;
+            if (w[k] & 7)  // a move that wrapped (grid edges)
+                q2 = add(load3(P.p.x, P.p.y, P.p.z, gj),
+                         image_translation(L.sT, code, w[k] & 1, (w[k] >> 1) & 1, (w[k] >> 2) & 1));
+            d[k] = sub(q2, v3(L.plan[m[k]], L.plan[M + m[k]], L.plan[2 * M + m[k]]));
+            in[k] = ((use >> k) & 1) && valid && j != (w[k] >> 8) && dot(d[k], d[k]) < K.range2;
+            any = any || in[k];
+        }
+        if (!__any(any)) continue;
+        if (!haveAxis) {
+            // most units out of the near shell have no entry within range: the orientations are read when one has
+            haveAxis = true;
+            double r[3];
+            for (int c = 0; c < 3; c++)
+                r[c] = fma(P.p.o[3 * c + 2][gj], K.axis.z,
+                           fma(P.p.o[3 * c + 1][gj], K.axis.y, P.p.o[3 * c][gj] * K.axis.x));
+            a2 = v3(r[0], r[1], r[2]);
+        }
+#pragma unroll
+        for (int k = 0; k < POLY_BATCH; k++) {
+            const double *ax = L.plan + 12 * M + m[k];
+            const bool keep = in[k] && !capsules_apart(K.halfLen, K.skip2, d[k], v3(ax[0], ax[M], ax[2 * M]), a2);
+            queued = poly_queue(keep, gj, (code << 6) | m[k], queue, queued);
+        }
+        queued = poly_make_room(P, K, L, queue, queued, own0, nOwn);
+    }
+    return queued;
+}
+
+// Scans the stencil for the moves of `active` and tests their trial poses against those of `undecided`: the own cell and
+// its neighbours first, where most of the moves of a dense packing end, then the other cells for the moves that overlap
+// nothing so far.  Returns the moves tested against the whole stencil.
+template <int WAVES>
+__device__ __forceinline__ unsigned long long poly_scan(const SweepParams &P, const PolyConsts &K, const Stencil &S, const PolyLds &L,
+                                          int own0, int nOwn, int total, unsigned long long active,
+                                          unsigned long long undecided) {
+    constexpr int M = POLY_MOVES;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    int *queue = L.queue + wave * 2 * POLY_QUEUE;
+    const int units = (total + WAVE - 1) / WAVE;
+    const int nearUnits = S.ncells > 27 ? min(units, (S.start[27] + WAVE - 1) / WAVE) : units;
+    int queued = 0, unit0 = 0;
+    unsigned long long left = active;
+    for (int shell = 0; shell < 2; shell++) {
+        const int unit1 = shell ? units : nearUnits;
+        queued = poly_units(P, K, S, L, own0, nOwn, total, unit0, unit1, left, wave, WAVES, queue, queued);
+        unit0 = unit1;
+        if (shell == 0 && __popcll(undecided) > 1) {
+            // the trial poses of moves a < m, one of them of this scan
+            for (int i = threadIdx.x; i < M * M; i += WAVE * WAVES) {
+                const int a = i & (M - 1), m = i / M;
+                const unsigned long long both = (1ull << a) | (1ull << m);
+                bool keep = false;
+                int code = 0;
+                if (a < m && (undecided & both) == both && (active & both)) {
+                    const int wa = L.word[a], wm = L.word[m];
+                    if ((wa >> 8) != (wm >> 8)) {
+                        code = wrap_code((unsigned)wa & 7);
+                        const double *qa = L.plan + a, *qm = L.plan + m;
+                        const V3 q2 = add(v3(qa[0], qa[M], qa[2 * M]),
+                                          image_translation(L.sT, code, wm & 1, (wm >> 1) & 1, (wm >> 2) & 1));
+                        const V3 d = sub(q2, v3(qm[0], qm[M], qm[2 * M]));
+                        keep = dot(d, d) < K.range2 &&
+                               !capsules_apart(K.halfLen, K.skip2, d, v3(qm[12 * M], qm[13 * M], qm[14 * M]),
+                                               v3(qa[12 * M], qa[13 * M], qa[14 * M]));
+                    }
+                }
+                queued = poly_queue(keep, -1 - a, (code << 6) | m, queue, queued);
+                queued = poly_make_room(P, K, L, queue, queued, own0, nOwn);
+            }
+        }
+        if (threadIdx.x % WAVE == 0) L.queued[wave] = queued;
+        queued = 0;
+        __syncthreads();
+        poly_drain<WAVES>(P, K, L, own0, nOwn);
+        if (unit0 >= units) break;
+        __syncthreads();
+        // (the same in every wavefront: nothing writes these until the next barrier)
+        const int lane = threadIdx.x & (WAVE - 1);
+        left = active & ~lds_mask2(L.hitOut) & __ballot(!(L.ownHit[2 * lane] | L.ownHit[2 * lane + 1]));
+        if (!left) break;
+        __syncthreads();
+    }
+    return unit0 < units ? 0ull : left;
+}
+
+// The trial pose of this lane's move i (its proposal) of own particle kIdx, from the records: the plan, and its word.
+__device__ __forceinline__ int poly_plan(const SweepParams &P, const PolyConsts &K, const PolyLds &L, int lane, int i,
+                                         int kIdx, int own0, int cell) {
+    constexpr int M = POLY_MOVES;
+    const int gi = own0 + kIdx;
+    double *q = L.plan + lane;
+    // Shape::rotate (Shape.cpp:14-16), the sums of mulm, a row at a time: few values live at once
+    {
+        double O[9];
+        for (int c = 0; c < 9; c++) O[c] = P.p.o[c][gi];
+        double ax[3];
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            double R[3], N[3];
+            for (int c = 0; c < 3; c++) R[c] = P.pr.R[(3 * r + c) * P.pr.stride + i];
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                double v = 0;
+                v += R[0] * O[c];
+                v += R[1] * O[3 + c];
+                v += R[2] * O[6 + c];
+                N[c] = v;
+                q[(3 + 3 * r + c) * M] = v;
+            }
+            ax[r] = fma(N[2], K.axis.z, fma(N[1], K.axis.y, N[0] * K.axis.x));
+        }
+        for (int c = 0; c < 3; c++) q[(12 + c) * M] = ax[c];
+    }
+    const V3 pos = load3(P.p.x, P.p.y, P.p.z, gi);
+    const V3 npos = translate_wrapped(L.box, L.box + 9, pos, v3(P.pr.t[i], P.pr.t[P.pr.stride + i],
+                                                                P.pr.t[2 * P.pr.stride + i]));
+    int nc[3];
+    unsigned nw;
+    bin_shifted(L.box + 9, L.box + 18, P.g.n, npos, nc, nw);
+    const bool inside = cell_index(P.g, nc[0], nc[1], nc[2]) == cell;
+    q[0] = npos.x;
+    q[M] = npos.y;
+    q[2 * M] = npos.z;
+    const int word = (inside ? (int)nw | 8 : 0) | (kIdx << 8);
+    L.word[lane] = word;
+    return word;
+}
+
+template <int WAVES>
+__device__ __forceinline__ void sweep_cell_poly(const SweepParams &P, const Stencil &S, const PolyLds &L, int own0, int nOwn,
+                                                int total, int cell) {
+    constexpr int M = POLY_MOVES, NT = WAVE * WAVES;
+    const int tid = threadIdx.x;
+    const int lane = tid & (WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int moves = P.moves > 0 ? P.moves : nOwn * P.mult;
+    const int pbase = P.moves > 0 ? cell * P.moves : own0 * P.mult;
+    unsigned long long accepted = 0, leftCell = 0, tests = 0;
+    unsigned long long tScan = 0, tRescan = 0, tDecide = 0, nRescans = 0;  // phase timers
+    PolyConsts K;
+    K.range2 = P.k.range2;
+    K.skip2 = P.skip2;
+    K.halfLen = P.k.capHalf;
+    K.axis = v3(P.k.capAxis[0], P.k.capAxis[1], P.k.capAxis[2]);
+    K.groupSize = P.k.groupSize;
+    K.groups = (P.k.nc + K.groupSize - 1) / K.groupSize;
+    K.pairShift = P.k.nc <= POLY_GROUPS ? 2 : 4;
+    K.pairs = WAVE >> K.pairShift;
+    for (int chunk = 0; chunk < moves; chunk += M) {
+        const int cn = min(M, moves - chunk);
+        // wavefront 0, a lane per move: the plan's word, the own particles overlapped, and whether the plan is stale
+        int word = 0, kIdx = 0;
+        bool stale = lane < cn;  // every move is planned first
+        bool again = false;      // to be scanned again as it is
+        int cur = 0;
+        unsigned long long accMask = 0, done = 0;  // done: tested against the whole stencil
+        for (int i = tid; i < POLY_RESULTS; i += NT) L.ownHit[i] = 0;
+        if (wave == 0 && lane < cn) kIdx = P.pr.k[pbase + chunk + lane];
+        __syncthreads();
+        for (int round = 0;; round++) {
+            if (wave == 0) {
+                if (stale) word = poly_plan(P, K, L, lane, pbase + chunk + lane, kIdx, own0, cell);
+                const unsigned long long scan = __ballot((stale || again) && (word & 8));
+                const unsigned long long out = lds_mask2(L.hitOut);
+                const unsigned long long undecided =
+                    __ballot(lane >= cur && lane < cn && (word & 8) && !((out >> lane) & 1));
+                stale = false;
+                if (lane < 2) {
+                    L.scan[lane] = (unsigned)(scan >> (32 * lane));
+                    L.undecided[lane] = (unsigned)(undecided >> (32 * lane));
+                }
+            }
+            __syncthreads();  // the plans; the records as of the last accepted moves
+            const unsigned long long tc0 = P.phases ? wall_clock64() : 0;
+            const unsigned long long active = lds_mask2(L.scan), undecided = lds_mask2(L.undecided);
+            // trial bead centres npos + NO c (PolysphereTraits.cpp:93-95), and the centres of the bead groups
+            for (int i = tid; i < M * (RP_MAX_CENTRES + POLY_GROUPS); i += NT) {
+                const int m = i & (M - 1), b = i / M, g = b - RP_MAX_CENTRES;
+                if (!((active >> m) & 1) || (g < 0 ? b / POLY_SLOTS : g) >= K.groups) continue;
+                const double *c = g < 0 ? L.beads + 4 * b : L.group + 4 * g;
+                double *q = L.plan + m;
+                double NO[9];
+                for (int e = 0; e < 9; e++) NO[e] = q[(3 + e) * M];
+                const V3 c1 = add(v3(q[0], q[M], q[2 * M]), mulv(NO, v3(c[0], c[1], c[2])));
+                q[(15 + 3 * b) * M] = c1.x;
+                q[(16 + 3 * b) * M] = c1.y;
+                q[(17 + 3 * b) * M] = c1.z;
+            }
+            __syncthreads();
+            const unsigned long long scanned = poly_scan<WAVES>(P, K, S, L, own0, nOwn, total, active, undecided);
+            __syncthreads();  // every hit of this scan is in LDS
+            const unsigned long long tc1 = P.phases ? wall_clock64() : 0;
+            if (P.phases) {
+                tScan += round ? 0 : tc1 - tc0;
+                tRescan += round ? tc1 - tc0 : 0;
+                nRescans += round ? 1 : 0;
+            }
+            if (wave == 0) {
+                unsigned mLo = L.ownHit[2 * lane], mHi = L.ownHit[2 * lane + 1];
+                const unsigned ttLo = L.tt[2 * lane], ttHi = L.tt[2 * lane + 1];
+                const unsigned long long out = lds_mask2(L.hitOut);
+                const bool alive = lane < cn && (word & 8) && !((out >> lane) & 1);
+                done = (done & ~active) | scanned;
+                unsigned long long staleMask = 0, againMask = 0;
+                for (;;) {
+                    const bool free = alive && !(mLo | mHi);
+                    staleMask = __ballot(stale);
+                    againMask = __ballot(lane >= cur && free && !stale) & ~done;
+                    const unsigned long long ev = __ballot(lane >= cur && (stale || free));
+                    if (!ev) {
+                        staleMask = againMask = 0;
+                        break;
+                    }
+                    const int a = __builtin_ctzll(ev);
+                    cur = a;
+                    // a stale move is planned and scanned again, one that an own particle alone had stopped is scanned
+                    // to the end, each with the others of its kind
+                    if (((staleMask | againMask) >> a) & 1) break;
+                    // accept move a (Packing::acceptMove: the cell belongs to this workgroup for the whole pass)
+                    const int wa = __builtin_amdgcn_readlane(word, a), ka = wa >> 8, gi = own0 + ka;
+                    accMask |= 1ull << a;
+                    if (lane < 13) {
+                        const double *q = L.plan + a;
+                        if (lane < 3) {
+                            double *dst = lane == 0 ? P.p.x : lane == 1 ? P.p.y : P.p.z;
+                            dst[gi] = q[lane * M];
+                        } else if (lane < 12) {
+                            P.p.o[lane - 3][gi] = q[lane * M];
+                        } else {
+                            P.p.wbits[gi] = (uint8_t)(wa & 7);
+                        }
+                    }
+                    // later moves: those of this particle are stale; the others meet its new pose
+                    if (lane > a && lane < cn) {
+                        if (kIdx == ka) {
+                            stale = true;
+                        } else {
+                            const unsigned bit = 1u << (ka & 31), now = ((a < 32 ? ttLo : ttHi) >> (a & 31)) & 1 ? bit : 0u;
+                            if (ka < 32) mLo = (mLo & ~bit) | now;
+                            else mHi = (mHi & ~bit) | now;
+                        }
+                    }
+                    cur = a + 1;
+                }
+                // the next scan ORs into these: the stale moves start anew, the others keep their results
+                L.ownHit[2 * lane] = stale ? 0 : mLo;
+                L.ownHit[2 * lane + 1] = stale ? 0 : mHi;
+                L.tt[2 * lane] = stale ? 0 : ttLo & ~(unsigned)staleMask;
+                L.tt[2 * lane + 1] = stale ? 0 : ttHi & ~(unsigned)(staleMask >> 32);
+                again = (againMask >> lane) & 1;
+                if (lane < 2) {
+                    L.hitOut[lane] = (unsigned)((out & ~staleMask) >> (32 * lane));
+                    L.more[lane] = (unsigned)((staleMask | againMask) >> (32 * lane));
+                }
+            }
+            if (P.phases) tDecide += wall_clock64() - tc1;
+            __syncthreads();
+            if (!lds_mask2(L.more)) break;
+        }
+        if (wave == 0) {
+            const int in = __popcll(__ballot(lane < cn && (word & 8)));
+            accepted += (unsigned long long)__popcll(accMask);
+            leftCell += (unsigned long long)(cn - in);
+            tests += (unsigned long long)total * (unsigned long long)in;
+            if (P.pr.acc && lane < cn && ((accMask >> lane) & 1)) P.pr.acc[pbase + chunk + lane] = 1;
+        }
+        __syncthreads();  // every wavefront has read `more` before the next chunk
+    }
+    if (P.phases && tid == 0) {
+        atomicAdd(&P.phases[RP_PHASE_PLAN], tScan);
+        atomicAdd(&P.phases[RP_PHASE_SCAN], tRescan);
+        atomicAdd(&P.phases[RP_PHASE_DECIDE], tDecide);
+        atomicAdd(&P.phases[RP_PHASE_GROUPS], accepted);
+        atomicAdd(&P.phases[RP_PHASE_REPLANS], nRescans);
+    }
+    flush_counters(P, cell, accepted, moves, leftCell, tests, true);
+}
+
 // Soft sweep of one active cell (Packing::tryMove with a soft interaction, Packing.cpp:136-164, and the Metropolis
 // test of Simulation.cpp:483).  In overlap-counting mode (Packing::calculateMoveOverlapEnergy, Packing.cpp:304-323)
 // the summed pair value is the overlap indicator, the move is accepted if it stays in the cell and its overlap
@@ -3099,7 +3630,34 @@ __device__ __forceinline__ void sweep_block(const SweepParams &P, const int b) {
     // with one cell across an axis the own cell recurs in its stencil under other images; staged copies would go
     // stale as particles move, so such grids read the stencil from HBM
     const bool ownRecurs = g.n[0] == 1 || g.n[1] == 1 || g.n[2] == 1;
-    if constexpr (LEAN != 0) {
+    if constexpr (LEAN != 0 && KIND == 2) {
+        const PolyLds L = carve_poly(smem);
+        for (int i = tid; i < 81; i += NT) L.sT[i] = g.T[i];
+        if (tid < 21) L.box[tid] = tid < 9 ? g.dims[tid] : tid < 18 ? g.inv[tid - 9] : g.shift[tid - 18];
+        for (int i = tid; i < 4 * (RP_MAX_CENTRES + POLY_GROUPS); i += NT) L.beads[i] = P.k.groups[i];
+        __syncthreads();
+        if (P.phases) clk[2] = wall_clock64();
+        if (nOwn <= OWN_CAP && !ownRecurs) {
+            sweep_cell_poly<WAVES>(P, S, L, own0, nOwn, total, cell);
+        } else {
+            // proposals in the area of the plans
+            static_assert(POLY_PLAN * POLY_MOVES >= 12 * MOVE_CHUNK && POLY_MOVES >= MOVE_CHUNK, "areas");
+            sweep_cell_unstaged<KIND, WAVES>(P, S, L.plan, L.plan + 3 * MOVE_CHUNK, L.word, L.sT, cell, own0, nOwn, total,
+                                             L.box, L.box + 9, L.box + 18);
+        }
+        if (P.phases) clk[3] = wall_clock64();
+        if (P.phases && tid == 0) {
+            clk[4] = wall_clock64();
+            atomicAdd(&P.phases[RP_PHASE_TABLE], clk[1] - clk[0]);
+            atomicAdd(&P.phases[RP_PHASE_STAGE], clk[2] - clk[1]);
+            atomicAdd(&P.phases[RP_PHASE_MOVES], clk[3] - clk[2]);
+            atomicAdd(&P.phases[RP_PHASE_WRITE], clk[4] - clk[3]);
+            atomicAdd(&P.phases[RP_PHASE_BLOCKS], 1ull);
+            atomicMax(&P.phases[RP_PHASE_LAST], clk[4] - clk[0]);
+        }
+        if (P.trace && tid == 0) trace_block(P, b, t0, nOwn, total, cell);
+        return;
+    } else if constexpr (LEAN != 0) {
         const SpecLds L = carve_spec<KIND, WAVES>(rest, P.cap);
         for (int i = tid; i < 81; i += NT) {
             L.sT[i] = g.T[i];
@@ -3735,7 +4293,7 @@ hipError_t launch_count_allpairs(hipStream_t s, const Grid &g, int n, Particles 
 int sweep_lean_cap() { return SPEC_CAP; }
 
 bool sweep_is_lean(const PairConsts &k, int waves, int pipelined, bool counting) {
-    return waves == 8 && pipelined == 2 && !k.soft && !counting && k.kind == 1;
+    return !k.soft && !counting && ((k.kind == 2 && waves >= 4) || (waves == 8 && pipelined == 2 && k.kind == 1));
 }
 
 int sweep_occupancy(int kind, int cap, int waves) {
@@ -3792,6 +4350,15 @@ hipError_t launch_sweep(hipStream_t s, const SweepParams &sp, int waves, Timed t
     if (g32 && (w != 8 || sp.pipelined != 2 || sp.fixMode || sp.k.kind != 1)) return hipErrorInvalidValue;
     const bool lean = !sp.fixMode && sweep_is_lean(sp.k, w, sp.pipelined, sp.counting != 0);
     size_t lds = sweep_lds_bytes(sp.k.kind, sp.cap, w, g32, lean);
+    if (lean && sp.k.kind == 2) {
+#define RP_SWEEP_P(W) \
+    hipExtLaunchKernelGGL((k_sweep<2, W, false, 1>), dim3(blocks), dim3(WAVE * W), (uint32_t)lds, s, t.start, t.stop, 0, sp)
+        if (w == 16) RP_SWEEP_P(16);
+        else if (w == 8) RP_SWEEP_P(8);
+        else RP_SWEEP_P(4);
+#undef RP_SWEEP_P
+        return hipGetLastError();
+    }
     if (lean) {
 #define RP_SWEEP_L(L) \
     hipExtLaunchKernelGGL((k_sweep<1, 8, false, L>), dim3(blocks), dim3(WAVE * 8), (uint32_t)lds, s, t.start, t.stop, 0, sp)
@@ -3810,11 +4377,9 @@ hipError_t launch_sweep(hipStream_t s, const SweepParams &sp, int waves, Timed t
     else if (w == 2) RP_SWEEP(KIND, 2, SOFT); \
     else RP_SWEEP(KIND, 1, SOFT);
     if (sp.k.kind == 2) {
-        // polyspheres: the hard sweep reading the stencil from HBM; counting mode through the soft sweep's counting
-        // branch (at most four wavefronts)
+        // polyspheres: counting mode through the soft sweep's counting branch (at most four wavefronts); the orientation
+        // fix on four wavefronts and the moves on one or two, one at a time
         if (sp.counting) { RP_SWEEP_W(2, true) }
-        else if (w == 16) RP_SWEEP(2, 16, false);
-        else if (w == 8) RP_SWEEP(2, 8, false);
         else { RP_SWEEP_W(2, false) }
     } else if (sp.k.kind == 0) {
         if (sp.k.soft || sp.counting) { RP_SWEEP_W(0, true) }

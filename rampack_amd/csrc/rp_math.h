@@ -177,6 +177,10 @@ struct PairConsts {
     int nc;              // polysphere: beads per particle
     const double *beads; // polysphere: device array, per bead body-frame x, y, z and radius
     double bound;        // polysphere: max over beads of |centre| + radius, rounded up (bounding-sphere radius)
+    // polysphere sweep (rp_create): the beads in groups of groupSize consecutive ones along the particle's long axis
+    const double *groups;  // device array: four bead slots (as above) for each of four groups, their bounding spheres
+    int groupSize;
+    double capAxis[3], capHalf, capRadius;  // a capsule about the centre that holds every bead (rounded up)
 };
 
 // Spherocylinder first-particle data that does not depend on the candidate.
