@@ -23,7 +23,7 @@ def run(beads, n_side, spacing, step, samplers, waves, cycles, monkeypatch):
     pk = ra.GpuPacking(shape(beads), box, pos, rot, seed=91)
     pk.set_environment(1.0, 1.0, step, None, box_move=("log", 0.002))
     if samplers > 1:
-        pk.set_move_samplers([("rototranslation", step, step)] * samplers)
+        pk.set_move_samplers([("rototranslation", (step, step))] * samplers)
     c = pk.run_cycles(cycles)
     out = pk.download()
     pk.close()
