@@ -415,22 +415,27 @@ __global__ __launch_bounds__(256) void k_bin(Grid g, int n, Particles src, int r
     }
     // The particles arrive in the previous grid's cell order, so a wavefront's lanes fall into a few cells: one
     // counter update per distinct cell, each lane's slot its rank among the lanes of that cell.  (Slots order the
-    // members only until the gather, which ranks them by source index.)
+    // members only until the gather, which ranks them by source index.)  The cells' updates are issued together once the
+    // ranks are known: one after another, their latencies add up where cells hold about one particle (1000 spheres: 32.5
+    // us with an update per pass of the loop, 7 so).
     unsigned long long active = __ballot(valid);
-    int slot = 0;
+    int leaderLane = 0, rank = 0, members = 0;
     while (active) {
         const int leader = __ffsll((long long)active) - 1;
         const int lc = __builtin_amdgcn_readlane(cell, leader);
         const unsigned long long same = __ballot(valid && cell == lc);
-        int base = 0;
-        if ((int)(threadIdx.x & (WAVE - 1)) == leader) base = atomicAdd(&g.cellCount[lc], (int)__popcll(same));
-        base = __builtin_amdgcn_readlane(base, leader);
-        if (valid && cell == lc)
-            slot = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(same >> 32),
-                                                         __builtin_amdgcn_mbcnt_lo((unsigned)same, 0u));
+        if (valid && cell == lc) {
+            leaderLane = leader;
+            members = (int)__popcll(same);
+            rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(same >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((unsigned)same, 0u));
+        }
         active &= ~same;
     }
-    if (valid) tmpSlot[i] = slot;
+    int base = 0;
+    if (valid && rank == 0) base = atomicAdd(&g.cellCount[cell], members);
+    base = __shfl(base, leaderLane);
+    if (valid) tmpSlot[i] = base + rank;
 }
 
 // Exclusive scan of the cell counts into cellStart (and cellStart[ncell] = n); the counts are cleared for the next
