@@ -679,22 +679,29 @@ __constant__ unsigned char kShellOrder[125] = {
     100, 101, 102, 103, 104, 105, 106, 107, 108, 109, 110, 111, 112, 113, 114, 115, 116, 117, 118, 119, 120, 121, 122, 123, 124
 };
 
-__device__ __forceinline__ void stencil_table(const Grid &g, int cx, int cy, int cz, int slot, bool half,
-                                              int *s_start, int *s_base, int *s_ecode, bool byShell = false) {
+// Slot `slot` of the stencil of cell (cx, cy, cz): the cell and its packed image shift (ecode).
+__device__ __forceinline__ int stencil_neighbour(const Grid &g, int cx, int cy, int cz, int slot, bool half, bool byShell,
+                                                 int &ecode) {
     const int k = g.reach, side = 2 * k + 1, centre = (side * side * side - 1) / 2;
     int t;
-    if (slot == 0) t = centre;
-    else if (half) t = centre + slot;
+    if (slot == 0 || half) t = centre + slot;
     else if (byShell && k == 2) t = kShellOrder[slot];
     else t = slot <= centre ? slot - 1 : slot;
     int ex, ey, ez;
     int nx = wrap_axis(cx, t / (side * side) - k, g.n[0], ex);
     int ny = wrap_axis(cy, (t / side) % side - k, g.n[1], ey);
     int nz = wrap_axis(cz, t % side - k, g.n[2], ez);
-    int nc = cell_index(g, nx, ny, nz);
+    ecode = (ex + 1) | ((ey + 1) << 2) | ((ez + 1) << 4);
+    return cell_index(g, nx, ny, nz);
+}
+
+__device__ __forceinline__ void stencil_table(const Grid &g, int cx, int cy, int cz, int slot, bool half,
+                                              int *s_start, int *s_base, int *s_ecode, bool byShell = false) {
+    int ecode;
+    const int nc = stencil_neighbour(g, cx, cy, cz, slot, half, byShell, ecode);
     s_base[slot] = g.cellStart[nc];
     s_start[slot + 1] = g.cellStart[nc + 1] - g.cellStart[nc];
-    s_ecode[slot] = (ex + 1) | ((ey + 1) << 2) | ((ez + 1) << 4);
+    s_ecode[slot] = ecode;
 }
 
 // Builds the table of `ncells` stencil cells and its prefix sums (s_start[ncells] = total entries).
@@ -732,7 +739,6 @@ __device__ __forceinline__ void stage_stencil(const Particles &p, const Stencil 
             S.ay[j] = p.o[5][gi];
             S.az[j] = p.o[8][gi];
         }
-        if (KIND == 2) S.ax[j] = (double)p.tag[gi];  // bead item index: particle * nc + bead
         S.code[j] = image_code(S.ecode[q], p.wbits[gi]);
     }
 }
@@ -744,7 +750,7 @@ __device__ __forceinline__ void carve_stencil(Stencil &S, double *smem, int cap,
     S.ax = S.z + cap;
     S.ay = S.ax + cap;
     S.az = S.ay + cap;
-    double *after = kind == 0 ? S.ax : S.az + cap;  // kind 2 keeps the bead item index in ax
+    double *after = kind == 0 ? S.ax : S.az + cap;
     S.code = reinterpret_cast<int *>(after);
     rest = after + (cap + 1) / 2;
 }
@@ -806,12 +812,10 @@ __device__ void count_cell(const Grid &g, const Particles &p, const PairConsts &
 constexpr int COUNT_OWN_CAP = 128;             // own particles whose first-operand data fits the table
 constexpr int COUNT_CHUNK = COUNT_THREADS * 8;  // pairs per chunk (and queue entries)
 
-// KIND 2 (bead items of polyspheres): pairs of beads of one particle are skipped (Packing.cpp:482-483, 500-501)
-// and the contact distance is the sum of the two bead radii (sBeadR, indexed by bead).
 template <int KIND>
 __device__ void count_cell_flat(const PairConsts &k, const Stencil &S, const double *sT, const int *sTag, int nOwn,
                                 int total, int earlyExit, unsigned long long *counters, int *sFound, double *fTab,
-                                int *queue, int *sQueued, const double *sBeadR) {
+                                int *queue, int *sQueued) {
     const int tid = threadIdx.x;
     const int lane = tid & (WAVE - 1);
     // first operands: position, cap A, u, a (10 doubles) per own particle
@@ -849,19 +853,10 @@ __device__ void count_cell_flat(const PairConsts &k, const Stencil &S, const dou
                     const int wx = (c1 & 3) - 1, wy = ((c1 >> 2) & 3) - 1, wz = ((c1 >> 4) & 3) - 1;
                     const V3 T = b < nOwn && code == c1 ? v3(0, 0, 0) : image_translation(sT, code, wx, wy, wz);
                     const double *q = fTab + 10 * a;
-                    if (KIND == 2) {
-                        const int ta = (int)S.ax[a], tb = (int)S.ax[b];
-                        const int pa = ta / k.nc, pb = tb / k.nc;
-                        if (pa != pb &&
-                            bead_overlap(sBeadR[ta - pa * k.nc], sBeadR[tb - pb * k.nc], v3(q[0], q[1], q[2]),
-                                         v3(S.x[b], S.y[b], S.z[b]), T))
-                            found++;
-                    } else {
-                        const V3 d = sub(add(v3(S.x[b], S.y[b], S.z[b]), T), v3(q[0], q[1], q[2]));
-                        const double d2 = dot(d, d);
-                        if (d2 < k.contact2) found++;
-                        else if (KIND == 1 && d2 < k.range2) amb = true;
-                    }
+                    const V3 d = sub(add(v3(S.x[b], S.y[b], S.z[b]), T), v3(q[0], q[1], q[2]));
+                    const double d2 = dot(d, d);
+                    if (d2 < k.contact2) found++;
+                    else if (KIND == 1 && d2 < k.range2) amb = true;
                 }
             }
             if (KIND == 1) {
@@ -930,20 +925,13 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count_overlaps(Grid g, Partic
     carve_stencil(S, smem, cap, KIND, rest);
     int *sTag = reinterpret_cast<int *>(rest);  // own-cell tags, up to cap entries
     for (int a = tid; a < nOwn && a < cap; a += COUNT_THREADS) sTag[a] = p.tag[own0 + a];
-    __shared__ double sBeadR[RP_MAX_CENTRES];
-    if (KIND == 2)
-        for (int c = tid; c < k.nc; c += COUNT_THREADS) sBeadR[c] = k.beads[4 * c + 3];
     if (total <= cap && nOwn <= COUNT_OWN_CAP && total <= 0xffff) {
         __shared__ int sQueued;
         stage_stencil<KIND>(p, S, total, tid, COUNT_THREADS);
         double *fTab = reinterpret_cast<double *>(sTag + ((cap + 1) & ~1));  // 10 doubles per own particle
         int *queue = reinterpret_cast<int *>(fTab + 10 * COUNT_OWN_CAP);        // COUNT_CHUNK entries
         __syncthreads();
-        count_cell_flat<KIND>(k, S, sT, sTag, nOwn, total, earlyExit, counters, &sFound, fTab, queue, &sQueued,
-                              sBeadR);
-    } else if (KIND == 2) {
-        // bead grids hold a few beads per cell; a cell beyond the flat path's limits is reported as an error
-        if (tid == 0) atomicAdd(&counters[CNT_STAGE_OVERFLOW], 1ull);
+        count_cell_flat<KIND>(k, S, sT, sTag, nOwn, total, earlyExit, counters, &sFound, fTab, queue, &sQueued);
     } else if (total <= cap) {
         stage_stencil<KIND>(p, S, total, tid, COUNT_THREADS);
         __syncthreads();
@@ -958,6 +946,77 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count_overlaps(Grid g, Partic
     if (tid == 0 && sFound) counters[CNT_SCAN_HINT] = (unsigned long long)cell;
 }
 
+// Overlap count of spheres (KIND 0) or bead items of polyspheres (KIND 2), COUNT_LANES lanes per item, each with one cell
+// of the item's half stencil (14 cells at reach 1), read in place.  Their grids hold about one item per cell, where a
+// workgroup per cell has a few busy lanes and most of its time is its launch.  Bound by the latency of its three dependent
+// reads (cell ranges, then items) at small sizes.  Pairs, their order and their translations are those of
+// count_cell_flat, and cells too full for its staging are reported in the same way.
+constexpr int COUNT_LANES = 16;
+template <int KIND>
+__global__ __launch_bounds__(COUNT_THREADS) void k_count_items(Grid g, int n, Particles p, PairConsts k, int earlyExit,
+                                                               unsigned long long *counters, int cap, int rot) {
+    __shared__ double sT[81], sBeadR[RP_MAX_CENTRES];
+    const int tid = threadIdx.x;
+    if (earlyExit && overlap_found(counters)) return;
+    for (int i = tid; i < 81; i += COUNT_THREADS) sT[i] = g.T[i];
+    if (KIND == 2)
+        for (int c = tid; c < k.nc; c += COUNT_THREADS) sBeadR[c] = k.beads[4 * c + 3];
+    __syncthreads();
+    // the items from those of cell `rot` on, then the ones before
+    const int at = (int)blockIdx.x * (COUNT_THREADS / COUNT_LANES) + tid / COUNT_LANES, sub = tid % COUNT_LANES;
+    const int ncells = stencil_cells(g.reach, true);
+    int found = 0, cell = 0, total = 0, own = 0;
+    if (at < n) {
+        int a = at + g.cellStart[rot];
+        if (a >= n) a -= n;
+        const V3 p1 = load3(p.x, p.y, p.z, a);
+        const int ta = p.tag[a], pa = KIND == 2 ? ta / k.nc : 0;
+        const double ra = KIND == 2 ? sBeadR[ta - pa * k.nc] : 0;
+        int c[3];
+        unsigned w;
+        bin_position(g, p1, c, w);  // as the rebuild binned it
+        cell = cell_index(g, c[0], c[1], c[2]);
+        const int wx = w & 1, wy = (w >> 1) & 1, wz = (w >> 2) & 1;
+        const int c1 = image_code(1 | (1 << 2) | (1 << 4), (int)w);
+        for (int slot = sub; slot < ncells && !(earlyExit && found); slot += COUNT_LANES) {
+            int ecode;
+            const int nc = stencil_neighbour(g, c[0], c[1], c[2], slot, true, false, ecode);
+            const int begin = g.cellStart[nc], end = g.cellStart[nc + 1];
+            total += end - begin;
+            if (slot == 0) own = end - begin;
+            if (KIND == 2 && end - begin > cap) continue;  // reported below
+            for (int b = begin; b < end; b++) {
+                const int tb = p.tag[b], pb = KIND == 2 ? tb / k.nc : 0;
+                // within the cell the item with the higher caller index is the first operand
+                if ((KIND == 2 && pa == pb) || (slot == 0 && tb >= ta)) continue;
+                const int code = image_code(ecode, p.wbits[b]);
+                const V3 T = slot == 0 && code == c1 ? v3(0, 0, 0) : image_translation(sT, code, wx, wy, wz);
+                const V3 p2 = load3(p.x, p.y, p.z, b);
+                bool hit;
+                if (KIND == 2) {
+                    hit = bead_overlap(ra, sBeadR[tb - pb * k.nc], p1, p2, T);
+                } else {
+                    const V3 d = rp::sub(add(p2, T), p1);
+                    hit = dot(d, d) < k.contact2;
+                }
+                found += hit ? 1 : 0;
+            }
+        }
+    }
+    for (int off = COUNT_LANES / 2; off > 0; off >>= 1) total += __shfl_xor(total, off);
+    // (lane 0 of the item has its own cell)
+    if (KIND == 0 ? own > cap : sub == 0 && (total > min(cap, 0xffff) || own > COUNT_OWN_CAP))
+        atomicAdd(&counters[CNT_STAGE_OVERFLOW], 1ull);
+    const unsigned long long any = __ballot(found != 0);
+    if (any) {
+        for (int off = WAVE / 2; off > 0; off >>= 1) found += __shfl_xor(found, off);
+        if ((tid & (WAVE - 1)) == __ffsll((long long)any) - 1) {
+            atomicAdd(&counters[CNT_OVERLAPS], (unsigned long long)found);
+            counters[CNT_SCAN_HINT] = (unsigned long long)cell;
+        }
+    }
+}
+
 size_t count_lds_bytes(int kind, int cap) {
     return stencil_lds_bytes(kind, cap) + sizeof(int) * (((cap + 1) & ~1) + COUNT_CHUNK) +
            sizeof(double) * 10 * COUNT_OWN_CAP;
@@ -968,14 +1027,19 @@ hipError_t launch_count_overlaps(hipStream_t s, const Grid &g, int n, Particles 
     if (n == 0) return hipSuccess;
     size_t lds = count_lds_bytes(k.kind, cap);
     const int rot = g.ncell > 0 ? ((startCell % g.ncell) + g.ncell) % g.ncell : 0;
-    if (k.kind == 0)
+    // spheres and beads in cells of a few: lanes per item
+    const unsigned perBlock = COUNT_THREADS / COUNT_LANES, items = ((unsigned)n + perBlock - 1) / perBlock;
+    if (k.kind == 2)
+        hipExtLaunchKernelGGL(k_count_items<2>, dim3(items), dim3(COUNT_THREADS), 0, s, t.start, t.stop, 0, g, n, p, k,
+                              earlyExit, counters, cap, rot);
+    else if (k.kind == 0 && n <= 4 * (long long)g.ncell)
+        hipExtLaunchKernelGGL(k_count_items<0>, dim3(items), dim3(COUNT_THREADS), 0, s, t.start, t.stop, 0, g, n, p, k,
+                              earlyExit, counters, cap, rot);
+    else if (k.kind == 0)
         hipExtLaunchKernelGGL(k_count_overlaps<0>, dim3((unsigned)g.ncell), dim3(COUNT_THREADS), (uint32_t)lds, s,
                               t.start, t.stop, 0, g, p, k, earlyExit, counters, cap, rot);
-    else if (k.kind == 1)
-        hipExtLaunchKernelGGL(k_count_overlaps<1>, dim3((unsigned)g.ncell), dim3(COUNT_THREADS), (uint32_t)lds, s,
-                              t.start, t.stop, 0, g, p, k, earlyExit, counters, cap, rot);
     else
-        hipExtLaunchKernelGGL(k_count_overlaps<2>, dim3((unsigned)g.ncell), dim3(COUNT_THREADS), (uint32_t)lds, s,
+        hipExtLaunchKernelGGL(k_count_overlaps<1>, dim3((unsigned)g.ncell), dim3(COUNT_THREADS), (uint32_t)lds, s,
                               t.start, t.stop, 0, g, p, k, earlyExit, counters, cap, rot);
     return hipGetLastError();
 }
