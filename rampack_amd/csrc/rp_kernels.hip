@@ -4078,7 +4078,7 @@ hipError_t launch_fix_all(hipStream_t s, const Particles &p, int n) {
 // Packings without a neighbour grid: every pair through the nearest image (PeriodicBoundaryConditions::getTranslation
 // for spherocylinders, getDistance2 for spheres; SpherocylinderTraits.cpp:28-46, SphereTraits.cpp:56-65)
 
-constexpr int ALLPAIRS_THREADS = 256;         // overlap count: a thread per particle
+constexpr int ALLPAIRS_THREADS = 256;         // overlap count: a wavefront per particle
 constexpr int ALLPAIRS_SWEEP_THREADS = 1024;  // sweep: one workgroup, the candidates of a move spread over its lanes
 constexpr int ALLPAIRS_CHUNK = 256;           // sweep: proposals staged in LDS at a time
 
@@ -4325,29 +4325,30 @@ __global__ __launch_bounds__(ALLPAIRS_SWEEP_THREADS) void k_sweep_allpairs_group
     flush_counters(P, cell, accepted, moves, 0, tests, true);
 }
 
+// A wavefront per particle i, its lanes over the candidates j: a thread per particle walked the candidates one after
+// another on two compute units (300 rods: 262 us, 7.3 so).
 template <int KIND>
 __global__ __launch_bounds__(ALLPAIRS_THREADS) void k_count_allpairs(Grid g, int n, Particles p, PairConsts k,
                                                                     int earlyExit, unsigned long long *counters) {
-    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) / WAVE), lane = threadIdx.x & (WAVE - 1);
     if (i >= n) return;
     const int ti = p.tag[i];
     const SCFirst f = make_first<KIND>(k, load3(p.x, p.y, p.z, i), v3(p.o[2][i], p.o[5][i], p.o[8][i]));
-    unsigned long long c = 0;
-    for (int j = 0; j < n; j++) {
+    int c = 0;
+    for (int j = lane; j < n && !(earlyExit && c); j += WAVE) {
         if (p.tag[j] <= ti) continue;  // each pair once, from the particle with the lower caller index
         const V3 a2 = KIND == 1 ? v3(p.o[2][j], p.o[5][j], p.o[8][j]) : v3(0, 0, 0);
-        if (allpairs_hit<KIND>(k, g, f, load3(p.x, p.y, p.z, j), a2)) {
-            c++;
-            if (earlyExit) break;
-        }
+        if (allpairs_hit<KIND>(k, g, f, load3(p.x, p.y, p.z, j), a2)) c++;
     }
-    if (c) atomicAdd(&counters[CNT_OVERLAPS], c);
+    if (!__any(c)) return;
+    for (int off = WAVE / 2; off > 0; off >>= 1) c += __shfl_xor(c, off);
+    if (lane == 0) atomicAdd(&counters[CNT_OVERLAPS], (unsigned long long)c);
 }
 
 hipError_t launch_count_allpairs(hipStream_t s, const Grid &g, int n, Particles p, PairConsts k, int earlyExit,
                                  unsigned long long *counters) {
     if (n == 0) return hipSuccess;
-    const unsigned blocks = (unsigned)((n + ALLPAIRS_THREADS - 1) / ALLPAIRS_THREADS);
+    const unsigned perBlock = ALLPAIRS_THREADS / WAVE, blocks = ((unsigned)n + perBlock - 1) / perBlock;
     if (k.kind == 0)
         hipLaunchKernelGGL(k_count_allpairs<0>, dim3(blocks), dim3(ALLPAIRS_THREADS), 0, s, g, n, p, k, earlyExit,
                            counters);
