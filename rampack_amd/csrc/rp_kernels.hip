@@ -4089,11 +4089,8 @@ __device__ __forceinline__ bool allpairs_hit(const PairConsts &k, const Grid &g,
     return sc_overlap(k, f, p2, a2, pbc_translation(g.dims, g.inv, f.pos, p2));
 }
 
-constexpr int AP_GROUP = 4;  // moves on distinct particles tested at once by the grouped all-pairs sweep
-
 size_t allpairs_lds_bytes(int n) {
-    return sizeof(double) * 12 * (size_t)n + (sizeof(double) * 12 + sizeof(int)) * ALLPAIRS_CHUNK +
-           sizeof(double) * 12 * AP_GROUP;
+    return sizeof(double) * 12 * (size_t)n + (sizeof(double) * 12 + sizeof(int)) * ALLPAIRS_CHUNK;
 }
 
 // The cycle's moves of a packing without a grid, in order, by one workgroup (Simulation::performMoves without domains,
@@ -4197,132 +4194,320 @@ __global__ __launch_bounds__(ALLPAIRS_SWEEP_THREADS) void k_sweep_allpairs(Sweep
     flush_counters(P, cell, accepted, moves, 0, tests, true);
 }
 
-// Grouped form of the staged all-pairs sweep: up to AP_GROUP consecutive moves on distinct particles are tested at
-// once against every particle and then decided in their order exactly as one at a time -- move k is rejected if it
-// overlaps a particle outside the group, the old pose of a group particle i not accepted before it (i > k, or i < k
-// rejected), or the trial pose of an accepted move i < k -- the rule of the grouped checkerboard sweep.  Same
-// decisions and trajectory as k_sweep_allpairs<KIND, true>; three barriers per group instead of one or two per move.
+// Speculative form of the all-pairs sweep, the scheme of sweep_cell_speculative with every particle an own one: a chunk of
+// 64 moves (a lane each in the deciding wavefront) is planned from the current poses and tested at once against every
+// particle and against the chunk's earlier trial poses; bit j of row m of `hit` says whether move m's trial pose overlaps
+// particle j in the pose it has now, bit a of tt[m] whether it overlaps move a's trial pose.  The first move without a hit
+// is accepted: its particle's bit of every later row becomes the row's bit of tt, and later moves of that particle are
+// stale, planned and tested again together when the first of them comes up.  Decisions and trajectory are those of one
+// move at a time.
+//
+// What bounds it: the FP64 arithmetic of the nearest images and segment tests on the one compute unit, then the chain of
+// accepted moves.  300 moves of a liquid of 300 rods: 249 us, 638 in groups of four moves with three barriers each.
+constexpr int AP_MOVES = 64;
+constexpr int AP_PLAN = 22;    // doubles per move: npos 3, its relative coordinates 3, NO 9, capA 3, u 3, a 1
+constexpr int AP_BATCH = 4;    // moves tested together
+constexpr int AP_QUEUE = WAVE + AP_BATCH * WAVE;  // pairs for the segment test per wavefront: drained to below 64
+
+struct AllPairsLds {
+    double *x, *y, *z, *ax, *ay, *az;  // the packing
+    double *plan;                      // AP_PLAN x AP_MOVES
+    unsigned *hit;                     // (n + 31) / 32 x AP_MOVES
+    unsigned *tt;                      // two words per move
+    unsigned *scan, *undecided, *more;  // two words each: see PolyLds
+    int *k;                            // particle of each move
+    int *queue;                        // per wavefront: particle (n + a: move a's trial pose) << 6 | move
+};
+
+size_t allpairs_spec_lds_bytes(int n) {
+    return sizeof(double) * (6 * (size_t)n + AP_PLAN * AP_MOVES) +
+           sizeof(int) * (AP_MOVES * (size_t)((n + 31) / 32 + 3) + 6 + ALLPAIRS_SWEEP_THREADS / WAVE * AP_QUEUE);
+}
+
+// pbc_translation with both positions' relative coordinates given (its own arithmetic from there on).
+__device__ __forceinline__ V3 nearest_translation(const double *dims, const V3 &a, const V3 &b) {
+    const double p[3] = {a.x, a.y, a.z}, q[3] = {b.x, b.y, b.z};
+    double t[3] = {0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        while (q[i] + t[i] - p[i] > 0.5) t[i] -= 1;
+        while (q[i] + t[i] - p[i] < -0.5) t[i] += 1;
+    }
+    return mulv(dims, v3(t[0], t[1], t[2]));
+}
+
+// Move m's trial pose against p2 (relative coordinates b2, axis a2): a certain hit, or a pair for the segment test.
 template <int KIND>
-__global__ __launch_bounds__(ALLPAIRS_SWEEP_THREADS) void k_sweep_allpairs_grouped(SweepParams P) {
+__device__ __forceinline__ void allpairs_near(const SweepParams &P, const AllPairsLds &L, int m, const V3 &p2, const V3 &b2,
+                                              const V3 &a2, bool &hit, bool &close) {
+    constexpr int M = AP_MOVES;
+    const double *q = L.plan + m;
+    const V3 pos = v3(q[0], q[M], q[2 * M]);
+    close = false;
+    if (KIND == 0) {
+        hit = pbc_distance2(P.g.dims, P.g.inv, pos, p2) < P.k.contact2;
+        return;
+    }
+    const V3 T = nearest_translation(P.g.dims, v3(q[3 * M], q[4 * M], q[5 * M]), b2);
+    const V3 d = sub(add(p2, T), pos);
+    const double d2 = dot(d, d);
+    hit = d2 < P.k.contact2;
+    close = !hit && d2 < P.k.range2 &&
+            !segments_apart(P.k.halfLen, P.skip2, d, v3(q[8 * M], q[11 * M], q[14 * M]), a2);
+}
+
+__device__ __forceinline__ void allpairs_mark(const AllPairsLds &L, int j, int m, int n) {
+    if (j < n) atomicOr(&L.hit[(j >> 5) * AP_MOVES + m], 1u << (j & 31));
+    else atomicOr(&L.tt[2 * m + ((j - n) >> 5)], 1u << ((j - n) & 31));
+}
+
+// Segment tests of at most 64 queued pairs.
+__device__ __forceinline__ void allpairs_segments(const SweepParams &P, const AllPairsLds &L, const int *entries, int count,
+                                                  int n) {
+    constexpr int M = AP_MOVES;
+    const int lane = threadIdx.x & (WAVE - 1);
+    __builtin_amdgcn_wave_barrier();  // the queue was written by other lanes of this wavefront
+    if (lane < count) {
+        const int e = entries[lane], j = e >> 6, m = e & (M - 1);
+        V3 p2, a2;
+        if (j < n) {
+            p2 = v3(L.x[j], L.y[j], L.z[j]);
+            a2 = v3(L.ax[j], L.ay[j], L.az[j]);
+        } else {
+            const double *q = L.plan + (j - n);
+            p2 = v3(q[0], q[M], q[2 * M]);
+            a2 = v3(q[8 * M], q[11 * M], q[14 * M]);
+        }
+        const double *q = L.plan + m;
+        const V3 T = nearest_translation(P.g.dims, v3(q[3 * M], q[4 * M], q[5 * M]), mulv(P.g.inv, p2));
+        const V3 c2 = add(p2, T);
+        if (segment_distance2(v3(q[15 * M], q[16 * M], q[17 * M]), v3(q[18 * M], q[19 * M], q[20 * M]), q[21 * M],
+                              add(c2, scal(a2, -P.k.halfLen)), add(c2, scal(a2, P.k.halfLen))) < P.k.contact2)
+            allpairs_mark(L, j, m, n);
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int KIND>
+__global__ __launch_bounds__(ALLPAIRS_SWEEP_THREADS) void k_sweep_allpairs_speculative(SweepParams P) {
     extern __shared__ double smem[];
-    __shared__ unsigned sHit[2];  // [0]: 5 bits per move (bit i < 4: old pose of member i, bit 4: outside the group)
-                                  // [1]: trial pairs, bit 4k + i: move k's trial pose overlaps move i's (i < k)
-    constexpr int T = ALLPAIRS_SWEEP_THREADS, C = ALLPAIRS_CHUNK, G = AP_GROUP;
+    constexpr int T = ALLPAIRS_SWEEP_THREADS, WAVES = T / WAVE, M = AP_MOVES;
     const Grid &g = P.g;
     const int cell = 0;  // the one cell of a packing without a grid
     const int n = g.cellStart[1];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int moves = P.moves;
     if (n > P.cap) {
         // the launch's LDS holds P.cap particles
         if (tid == 0) atomicAdd(&P.counters[CNT_STAGE_OVERFLOW], 1ull);
         return;
     }
-    double *sx = smem, *sy = sx + n, *sz = sy + n;
-    double *so = sz + n;  // component c of particle j at so[c * n + j]
-    double *ct = so + 9 * n, *cR = ct + 3 * C;
-    int *ck = (int *)(cR + 9 * C);
-    double *plan = (double *)(ck + C);  // per group member: trial position (3) and orientation (9)
+    const int words = (n + 31) / 32;
+    AllPairsLds L;
+    L.x = smem;
+    L.y = L.x + n;
+    L.z = L.y + n;
+    L.ax = L.z + n;
+    L.ay = L.ax + n;
+    L.az = L.ay + n;
+    L.plan = L.az + n;
+    L.hit = reinterpret_cast<unsigned *>(L.plan + AP_PLAN * M);
+    L.tt = L.hit + words * M;
+    L.scan = L.tt + 2 * M;
+    L.undecided = L.scan + 2;
+    L.more = L.undecided + 2;
+    L.k = reinterpret_cast<int *>(L.more + 2);
+    L.queue = L.k + M;
+    int *queue = L.queue + wave * AP_QUEUE;
     for (int j = tid; j < n; j += T) {
-        sx[j] = P.p.x[j];
-        sy[j] = P.p.y[j];
-        sz[j] = P.p.z[j];
-        for (int c = 0; c < 9; c++) so[c * n + j] = P.p.o[c][j];
+        L.x[j] = P.p.x[j];
+        L.y[j] = P.p.y[j];
+        L.z[j] = P.p.z[j];
+        L.ax[j] = P.p.o[2][j];
+        L.ay[j] = P.p.o[5][j];
+        L.az[j] = P.p.o[8][j];
     }
-    unsigned long long accepted = 0, tests = 0;
-    for (int base = 0; base < moves; base += C) {
-        const int cn = min(C, moves - base);
-        __syncthreads();  // the packing staged; every thread done with the previous chunk's proposals
-        if (tid < cn) {
-            const int i = base + tid;
-            ck[tid] = P.pr.k[i];
-            for (int d = 0; d < 3; d++) ct[d * C + tid] = P.pr.t[d * P.pr.stride + i];
-            for (int c = 0; c < 9; c++) cR[c * C + tid] = P.pr.R[c * P.pr.stride + i];
+    unsigned long long accepted = 0;
+    for (int chunk = 0; chunk < moves; chunk += M) {
+        const int cn = min(M, moves - chunk);
+        for (int i = tid; i < (words + 2) * M; i += T) L.hit[i] = 0;  // (tt follows the rows)
+        int kIdx = 0, cur = 0;
+        bool stale = wave == 0 && lane < cn;  // every move is planned first
+        unsigned long long accMask = 0;
+        if (stale) {
+            kIdx = P.pr.k[chunk + lane];
+            L.k[lane] = kIdx;
         }
-        __syncthreads();
-        for (int m0 = 0; m0 < cn;) {
-            // the group: the longest run of at most G moves on distinct particles (the same in every lane)
-            const int c0 = ck[m0];
-            const int c1 = m0 + 1 < cn ? ck[m0 + 1] : -1, c2 = m0 + 2 < cn ? ck[m0 + 2] : -1;
-            const int c3 = m0 + 3 < cn ? ck[m0 + 3] : -1;
-            const bool d1 = m0 + 1 < cn && c1 != c0;
-            const bool d2 = d1 && m0 + 2 < cn && c2 != c0 && c2 != c1;
-            const bool d3 = d2 && m0 + 3 < cn && c3 != c0 && c3 != c1 && c3 != c2;
-            const int gs = 1 + (int)d1 + (int)d2 + (int)d3;
-            const int k0 = c0, k1 = d1 ? c1 : -1, k2 = d2 ? c2 : -1, k3 = d3 ? c3 : -1;
-            auto kof = [&](int k) { return k == 0 ? k0 : (k == 1 ? k1 : (k == 2 ? k2 : k3)); };
-            if (tid < gs) {
-                // trial pose of move m0 + tid (Shape::translate with the periodic correction, Shape::rotate)
-                const int mm = m0 + tid, ki = kof(tid);
-                const V3 npos = translate_wrapped(g.dims, g.inv, v3(sx[ki], sy[ki], sz[ki]),
-                                                  v3(ct[mm], ct[C + mm], ct[2 * C + mm]));
-                double O[9], R[9], NO[9];
-                for (int c = 0; c < 9; c++) {
-                    O[c] = so[c * n + ki];
-                    R[c] = cR[c * C + mm];
+        __syncthreads();  // the rows cleared; the packing staged
+        for (;;) {
+            if (wave == 0) {
+                if (stale) {
+                    // trial pose (Shape::translate with the periodic correction, Shape::rotate) from the current pose
+                    const int i = chunk + lane;
+                    double *q = L.plan + lane;
+                    // the sums of mulm, a row at a time: few values live at once
+                    V3 nax;
+                    {
+                        double O[9];
+                        for (int c = 0; c < 9; c++) O[c] = P.p.o[c][kIdx];
+#pragma unroll
+                        for (int r = 0; r < 3; r++) {
+                            double R[3];
+                            for (int c = 0; c < 3; c++) R[c] = P.pr.R[(3 * r + c) * P.pr.stride + i];
+#pragma unroll
+                            for (int c = 0; c < 3; c++) {
+                                double v = 0;
+                                v += R[0] * O[c];
+                                v += R[1] * O[3 + c];
+                                v += R[2] * O[6 + c];
+                                q[(6 + 3 * r + c) * M] = v;
+                                if (c == 2) (r == 0 ? nax.x : r == 1 ? nax.y : nax.z) = v;
+                            }
+                        }
+                    }
+                    const V3 npos = translate_wrapped(g.dims, g.inv, v3(L.x[kIdx], L.y[kIdx], L.z[kIdx]),
+                                                      v3(P.pr.t[i], P.pr.t[P.pr.stride + i], P.pr.t[2 * P.pr.stride + i]));
+                    const V3 rel = mulv(g.inv, npos);
+                    q[0] = npos.x;
+                    q[M] = npos.y;
+                    q[2 * M] = npos.z;
+                    q[3 * M] = rel.x;
+                    q[4 * M] = rel.y;
+                    q[5 * M] = rel.z;
+                    if (KIND == 1) {
+                        const SCFirst f = sc_first(P.k, npos, nax);
+                        q[15 * M] = f.capA.x;
+                        q[16 * M] = f.capA.y;
+                        q[17 * M] = f.capA.z;
+                        q[18 * M] = f.u.x;
+                        q[19 * M] = f.u.y;
+                        q[20 * M] = f.u.z;
+                        q[21 * M] = f.a;
+                    }
                 }
-                mulm(R, O, NO);
-                double *q = plan + 12 * tid;
-                q[0] = npos.x;
-                q[1] = npos.y;
-                q[2] = npos.z;
-                for (int c = 0; c < 9; c++) q[3 + c] = NO[c];
+                const unsigned long long scan = __ballot(stale), undecided = __ballot(lane >= cur && lane < cn);
+                stale = false;
+                if (lane < 2) {
+                    L.scan[lane] = (unsigned)(scan >> (32 * lane));
+                    L.undecided[lane] = (unsigned)(undecided >> (32 * lane));
+                }
             }
-            if (tid < 2) sHit[tid] = 0;
+            __syncthreads();  // the plans
+            const unsigned long long active = lds_mask2(L.scan), undecided = lds_mask2(L.undecided);
+            const int batches = (__popcll(active) + AP_BATCH - 1) / AP_BATCH;
+            const int units = (n + WAVE - 1) / WAVE, items = units * batches;
+            int queued = 0;
+            auto take = [&](bool hit, bool close, int j, int m) {
+                if (hit) allpairs_mark(L, j, m, n);
+                if (KIND == 1) {
+                    const unsigned long long mask = __ballot(close);
+                    if (close)
+                        queue[queued + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                                                      __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u))] =
+                            (j << 6) | m;
+                    queued += __popcll(mask);
+                }
+            };
+            auto drain = [&]() {
+                while (queued >= WAVE) {
+                    queued -= WAVE;
+                    allpairs_segments(P, L, queue + queued, WAVE, n);
+                }
+            };
+            for (int item = items * wave / WAVES, last = items * (wave + 1) / WAVES; item < last; item++) {
+                const int unit = item / batches, batch = item - unit * batches;
+                unsigned long long rest = active;
+                for (int i = 0; i < batch * AP_BATCH; i++) rest &= rest - 1;
+                const int j = unit * WAVE + lane;
+                const bool valid = j < n;
+                const int jj = valid ? j : 0;
+                const V3 p2 = v3(L.x[jj], L.y[jj], L.z[jj]), a2 = v3(L.ax[jj], L.ay[jj], L.az[jj]);
+                const V3 b2 = mulv(g.inv, p2);
+                for (int i = 0; i < AP_BATCH && rest; i++, rest &= rest - 1) {
+                    const int m = __builtin_ctzll(rest);
+                    bool hit, close;
+                    allpairs_near<KIND>(P, L, m, p2, b2, a2, hit, close);
+                    const bool use = valid && j != L.k[m];
+                    take(use && hit, use && close, j, m);
+                }
+                drain();
+            }
+            // the trial poses of moves a < m, one of them of this scan
+            for (int i = tid; i < M * M; i += T) {
+                const int a = i & (M - 1), m = i / M;
+                const unsigned long long both = (1ull << a) | (1ull << m);
+                bool hit = false, close = false;
+                if (a < m && (undecided & both) == both && (active & both) && L.k[a] != L.k[m]) {
+                    const double *q = L.plan + a;
+                    allpairs_near<KIND>(P, L, m, v3(q[0], q[M], q[2 * M]), v3(q[3 * M], q[4 * M], q[5 * M]),
+                                        v3(q[8 * M], q[11 * M], q[14 * M]), hit, close);
+                }
+                take(hit, close, n + a, m);
+                drain();
+            }
+            if (queued > 0) allpairs_segments(P, L, queue, queued, n);
+            __syncthreads();  // every hit of this scan is in LDS
+            if (wave == 0) {
+                int hits = 0;
+                for (int w = 0; w < words; w++) hits += __popc(L.hit[w * M + lane]);
+                const unsigned ttLo = L.tt[2 * lane], ttHi = L.tt[2 * lane + 1];
+                unsigned long long staleMask = 0;
+                for (;;) {
+                    staleMask = __ballot(stale);
+                    const unsigned long long ev = __ballot(lane >= cur && lane < cn && (stale || hits == 0));
+                    if (!ev) {
+                        staleMask = 0;
+                        break;
+                    }
+                    const int a = __builtin_ctzll(ev);
+                    cur = a;
+                    if ((staleMask >> a) & 1) break;  // planned and scanned again with the other stale moves
+                    const int ka = __builtin_amdgcn_readlane(kIdx, a);
+                    accMask |= 1ull << a;
+                    const double *q = L.plan + a;
+                    if (lane < 3) {
+                        double *dst = lane == 0 ? P.p.x : lane == 1 ? P.p.y : P.p.z;
+                        dst[ka] = q[lane * M];
+                        (lane == 0 ? L.x : lane == 1 ? L.y : L.z)[ka] = q[lane * M];
+                    } else if (lane < 12) {
+                        P.p.o[lane - 3][ka] = q[(lane + 3) * M];
+                    } else if (lane < 15) {
+                        (lane == 12 ? L.ax : lane == 13 ? L.ay : L.az)[ka] = q[(8 + 3 * (lane - 12)) * M];
+                    } else if (lane == 15) {
+                        P.p.wbits[ka] = 0;
+                    }
+                    // later moves: those of this particle are stale; the others meet its new pose
+                    if (lane > a && lane < cn) {
+                        if (kIdx == ka) {
+                            stale = true;
+                        } else {
+                            unsigned *row = &L.hit[(ka >> 5) * M + lane];
+                            const unsigned old = *row, bit = 1u << (ka & 31);
+                            const unsigned now = ((a < 32 ? ttLo : ttHi) >> (a & 31)) & 1 ? old | bit : old & ~bit;
+                            hits += __popc(now) - __popc(old);
+                            *row = now;
+                        }
+                    }
+                    cur = a + 1;
+                }
+                // the next scan ORs into these: the stale moves start anew, the others keep their results
+                if (stale)
+                    for (int w = 0; w < words; w++) L.hit[w * M + lane] = 0;
+                L.tt[2 * lane] = stale ? 0 : ttLo & ~(unsigned)staleMask;
+                L.tt[2 * lane + 1] = stale ? 0 : ttHi & ~(unsigned)(staleMask >> 32);
+                if (lane < 2) L.more[lane] = (unsigned)(staleMask >> (32 * lane));
+            }
             __syncthreads();
-            unsigned hw = 0, tw = 0;
-            for (int k = 0; k < gs; k++) {
-                const double *q = plan + 12 * k;
-                const SCFirst f = make_first<KIND>(P.k, v3(q[0], q[1], q[2]), v3(q[5], q[8], q[11]));
-                const int kk = kof(k);
-                for (int j = tid; j < n; j += T) {
-                    if (j == kk) continue;
-                    const int member = j == k0 ? 0 : (j == k1 ? 1 : (j == k2 ? 2 : (j == k3 ? 3 : 4)));
-                    const unsigned bit = 1u << (5 * k + member);
-                    if (hw & bit) continue;
-                    const V3 a2 = KIND == 1 ? v3(so[2 * n + j], so[5 * n + j], so[8 * n + j]) : v3(0, 0, 0);
-                    if (allpairs_hit<KIND>(P.k, g, f, v3(sx[j], sy[j], sz[j]), a2)) hw |= bit;
-                }
-                // lanes 4k + i test move k's trial pose against move i's (i < k)
-                for (int i = 0; i < k; i++) {
-                    if (tid != 4 * k + i) continue;
-                    const double *qi = plan + 12 * i;
-                    const V3 a2 = KIND == 1 ? v3(qi[5], qi[8], qi[11]) : v3(0, 0, 0);
-                    if (allpairs_hit<KIND>(P.k, g, f, v3(qi[0], qi[1], qi[2]), a2)) tw |= 1u << (4 * k + i);
-                }
-            }
-            if (hw) atomicOr(&sHit[0], hw);
-            if (tw) atomicOr(&sHit[1], tw);
-            __syncthreads();
-            // the group's decisions in order (the same in every lane)
-            const unsigned H = sHit[0], TP = sHit[1];
-            unsigned acc = 0;
-            for (int k = 0; k < gs; k++) {
-                const unsigned b = (H >> (5 * k)) & 31u, trial = (TP >> (4 * k)) & 15u;
-                const bool hit = (b & 16u) || ((b & 15u) & ~acc) || (trial & acc);
-                if (!hit) acc |= 1u << k;
-            }
-            accepted += (unsigned long long)__popc(acc);
-            tests += (unsigned long long)(n - 1) * (unsigned long long)gs;
-            if (tid < gs && ((acc >> tid) & 1u)) {
-                const int ki = kof(tid);
-                const double *q = plan + 12 * tid;
-                P.p.x[ki] = q[0];
-                P.p.y[ki] = q[1];
-                P.p.z[ki] = q[2];
-                for (int c = 0; c < 9; c++) P.p.o[c][ki] = q[3 + c];
-                P.p.wbits[ki] = 0;
-                if (P.pr.acc) P.pr.acc[base + m0 + tid] = 1;
-                sx[ki] = q[0];
-                sy[ki] = q[1];
-                sz[ki] = q[2];
-                for (int c = 0; c < 9; c++) so[c * n + ki] = q[3 + c];
-            }
-            __syncthreads();  // accepted poses staged; the plan and hit words free for the next group
-            m0 += gs;
+            if (!lds_mask2(L.more)) break;
         }
+        if (wave == 0) {
+            accepted += (unsigned long long)__popcll(accMask);
+            if (P.pr.acc && lane < cn && ((accMask >> lane) & 1)) P.pr.acc[chunk + lane] = 1;
+        }
+        __syncthreads();  // every wavefront has read `more` before the next chunk
     }
-    flush_counters(P, cell, accepted, moves, 0, tests, true);
+    flush_counters(P, cell, accepted, moves, 0, (unsigned long long)(n - 1) * (unsigned long long)moves, true);
 }
 
 // A wavefront per particle i, its lanes over the candidates j: a thread per particle walked the candidates one after
@@ -4391,23 +4576,22 @@ hipError_t launch_sweep(hipStream_t s, const SweepParams &sp, int waves, Timed t
         // no grid: one workgroup runs the cycle's moves in order (hard spheres and spherocylinders)
         if (g32 || sp.k.soft || sp.counting || sp.k.kind == 2 || (!sp.fixMode && sp.moves <= 0))
             return hipErrorInvalidValue;
-        // sp.cap > 0: the packing (at most sp.cap particles) and the proposals staged in LDS
-        const uint32_t lds = sp.cap > 0 ? (uint32_t)allpairs_lds_bytes(sp.cap) : 0;
-#define RP_ALLPAIRS(KIND, STAGED) \
-    hipExtLaunchKernelGGL((k_sweep_allpairs<KIND, STAGED>), dim3(1), dim3(ALLPAIRS_SWEEP_THREADS), lds, s, t.start, t.stop, \
-                          0, sp)
-#define RP_ALLPAIRS_GROUPED(KIND) \
-    hipExtLaunchKernelGGL((k_sweep_allpairs_grouped<KIND>), dim3(1), dim3(ALLPAIRS_SWEEP_THREADS), lds, s, t.start, \
-                          t.stop, 0, sp)
-        // staged packings: grouped moves; the orientation fix and packings too large for LDS: one move at a time
-        const bool grouped = sp.cap > 0 && !sp.fixMode;
-        if (sp.k.kind == 0 && grouped) RP_ALLPAIRS_GROUPED(0);
-        else if (sp.k.kind == 0 && sp.cap > 0) RP_ALLPAIRS(0, true);
-        else if (sp.k.kind == 0) RP_ALLPAIRS(0, false);
-        else if (grouped) RP_ALLPAIRS_GROUPED(1);
-        else if (sp.cap > 0) RP_ALLPAIRS(1, true);
-        else RP_ALLPAIRS(1, false);
-#undef RP_ALLPAIRS_GROUPED
+        // sp.cap > 0: the packing (at most sp.cap particles) staged in LDS
+#define RP_ALLPAIRS(KERNEL, BYTES) \
+    hipExtLaunchKernelGGL(KERNEL, dim3(1), dim3(ALLPAIRS_SWEEP_THREADS), (uint32_t)(BYTES), s, t.start, t.stop, 0, sp)
+        // staged packings: speculative moves; the orientation fix and packings too large for LDS: one move at a time
+        if (sp.cap > 0 && !sp.fixMode) {
+            const size_t lds = allpairs_spec_lds_bytes(sp.cap);
+            if (sp.k.kind == 0) RP_ALLPAIRS((k_sweep_allpairs_speculative<0>), lds);
+            else RP_ALLPAIRS((k_sweep_allpairs_speculative<1>), lds);
+        } else if (sp.cap > 0) {
+            const size_t lds = allpairs_lds_bytes(sp.cap);
+            if (sp.k.kind == 0) RP_ALLPAIRS((k_sweep_allpairs<0, true>), lds);
+            else RP_ALLPAIRS((k_sweep_allpairs<1, true>), lds);
+        } else {
+            if (sp.k.kind == 0) RP_ALLPAIRS((k_sweep_allpairs<0, false>), 0);
+            else RP_ALLPAIRS((k_sweep_allpairs<1, false>), 0);
+        }
 #undef RP_ALLPAIRS
         return hipGetLastError();
     }
