@@ -1150,8 +1150,12 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
     int cap = (int)std::ceil(expect + 8 * std::sqrt(expect) + 64);
     cap = (cap + 63) / 64 * 64;
     int waves = c->sweepWaves;
-    // eight wavefronts with grouped moves for dense stencils (measured fastest on 1e5 rods), else fewer
-    if (waves <= 0) waves = expect > 384 ? 8 : (expect > 128 ? 2 : 1);
+    // Eight wavefronts for dense stencils, else fewer.  Hard spherocylinders take the eight of the speculative sweep from
+    // 180 particles per stencil on (200 cycles of 16 000 rods at 220: 48.6 ms against 53.6 on one wavefront, at 300 49.2
+    // against 75.5; 3 456 rods at 155: 45.1 against 43.7).  Two wavefronts with a planner, which ran at 128 to 384 before,
+    // faulted the GPU on layered packings with partly empty cells, and the cause is not found.
+    const bool hardRods = c->k.kind == RP_SHAPE_SPHEROCYLINDER && !c->k.soft && !c->counting && c->pipelined < 0;
+    if (waves <= 0) waves = hardRods ? (expect > 180 ? 8 : 1) : (expect > 384 ? 8 : (expect > 128 ? 2 : 1));
     // hard polyspheres: the speculative sweep on eight or sixteen wavefronts once a stencil holds some 200 particles, one
     // move at a time below that (10 cycles on 5-bead chains, stencils of 270: 14.8 ms against 17.2 with two wavefronts one
     // at a time; 3-bead chains, 130: 9.2 on four wavefronts against 7.7; 7-bead chains, 650: sixteen 16.0, eight 16.3)
@@ -1162,9 +1166,9 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
     if (waves == 16 && (c->k.kind != RP_SHAPE_POLYSPHERE || c->k.soft || c->counting)) waves = 8;
     // eight wavefronts only for the hard sweeps
     if (waves == 8 && (c->k.soft || c->counting)) waves = 4;
-    // per-sampler acceptance flags are compiled into the kernels of at most four wavefronts only (the eight-wavefront
-    // kernel has no registers to spare for them)
-    if (waves >= 8 && ms.n > 1 && c->k.kind != RP_SHAPE_POLYSPHERE) waves = 4;
+    // the eight-wavefront kernels that make one move at a time write no per-sampler acceptance flags (no registers to spare
+    // for them); the speculative sweeps do
+    if (waves >= 8 && ms.n > 1 && !hardRods && c->k.kind != RP_SHAPE_POLYSPHERE) waves = 4;
     sp.pipelined = c->pipelined >= 0 ? c->pipelined : (waves >= 8 ? 2 : 1);
     // guarded FP32 stencil scan: the default launch of hard spherocylinders (eight wavefronts, grouped moves); the
     // all-pairs path (no grid) tests in FP64
