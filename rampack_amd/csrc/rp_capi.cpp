@@ -1170,7 +1170,7 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
     // for them); the speculative sweeps do
     if (waves >= 8 && ms.n > 1 && !hardRods && c->k.kind != RP_SHAPE_POLYSPHERE) waves = 4;
     sp.pipelined = c->pipelined >= 0 ? c->pipelined : (waves >= 8 ? 2 : 1);
-    // guarded FP32 stencil scan: the default launch of hard spherocylinders (eight wavefronts, grouped moves); the
+    // guarded FP32 stencil scan: the default launch of hard spherocylinders (eight wavefronts, speculative moves); the
     // all-pairs path (no grid) tests in FP64
     const int g32 = c->precision != RP_PREC_FP64 && waves == 8 && sp.pipelined == 2 && !c->k.soft && !c->counting &&
                     c->k.kind == RP_SHAPE_SPHEROCYLINDER && !g.allPairs ? c->precision : 0;

@@ -70,7 +70,7 @@ struct SweepParams {
     int na[3];              // active cells per axis (n / period)
     int cap;                // stencil entries that fit in LDS; without a grid: the particles the all-pairs sweep
                             // stages in LDS (0: it reads them in place)
-    int pipelined;          // 1: wavefront 0 plans the next move while the others test; 2: grouped moves
+    int pipelined;          // 1: wavefront 0 plans the next move while the others test; 2: grouped or speculative moves
                             // (both need >= 2 wavefronts)
     double temperature;     // soft interactions: the move is accepted if u <= exp(-dE / temperature)
     int counting;           // overlap-counting mode (Packing::toggleOverlapCounting): a move is accepted if it does not
@@ -84,7 +84,7 @@ struct SweepParams {
                                  // that scan one slot more than the others
     unsigned long long *trace;   // optional per-workgroup record of one launch: start and end wall clock,
                                  // own | stencil << 16 | cell << 32, compute-unit id; nullptr when not tracing
-    // Guarded FP32 stencil scan of the grouped sweep (k_sweep<..., G32 = 1 or 2>): candidate positions relative to the
+    // Guarded FP32 stencil scan of the speculative sweep (G32 = 1 or 2): candidate positions relative to the
     // active cell's centre in FP32, squared centre distances in FP32, and the FP64 value only for pairs the FP32 value
     // cannot place on one side of a threshold.  g32Lim[s] = {contact2 lower, contact2 upper, range2 lower,
     // range2 upper} bounds of the FP32 guard bands, s = 0 for cells whose stencil was staged translated (no wrapped

@@ -8,11 +8,13 @@
 //                        NeighbourGrid insertion (Packing.cpp:858-929, NeighbourGrid.cpp:219-227); the order
 //                        inside a cell is the stable order of the source arrays, so rebuilds are deterministic
 //   * k_count_overlaps   half-shell overlap count with early exit (Packing.cpp:431-559), one workgroup per cell
-//                        with the cell and its 13 positive neighbours staged in LDS
-//   * k_sweep            checkerboard MC sweep: one workgroup (1, 2 or 4 wavefronts) per active cell, the 27-cell
-//                        stencil staged in LDS, early-exit overlap voting after every 64*waves candidates, a Philox
-//                        stream per move, moves that leave the cell rejected (the ActiveDomain rule of
-//                        Packing.cpp:147-148)
+//                        with the cell and its 13 positive neighbours staged in LDS; k_count_items: lanes per item,
+//                        for the sparse grids of spheres and beads
+//   * k_sweep            checkerboard MC sweep: one workgroup (1 to 16 wavefronts) per active cell, a Philox stream
+//                        per move, moves that leave the cell rejected (the ActiveDomain rule of
+//                        Packing.cpp:147-148).  Dense hard cells test all moves of a chunk against the stencil at
+//                        once and decide them in order (sweep_cell_speculative, sweep_cell_poly); the others make
+//                        one move, or a group of four, at a time
 #include "rp_kernels.h"
 
 #include <hip/hip_ext.h>
@@ -3654,9 +3656,9 @@ __device__ __forceinline__ void trace_block(const SweepParams &P, int b, unsigne
 }
 
 // Active cell b of colour P.colour (one workgroup).
-// LEAN != 0: the kernel carries only the grouped sweep of staged cells (and the HBM path for cells that cannot be
-// staged), with fewer live registers than the general kernel: 1 FP64 scan, 2 guarded FP32 scan, 3 guarded FP32 scan
-// with the FP64 verification of every pair.
+// LEAN != 0: the kernel carries only the speculative sweep of hard spherocylinders or polyspheres (and the HBM path for
+// cells that cannot take it), with fewer live registers than the general kernel: 1 FP64 scan, 2 guarded FP32 scan, 3
+// guarded FP32 scan with the FP64 verification of every pair.
 template <int KIND, int WAVES, bool SOFT, int LEAN>
 __device__ __forceinline__ void sweep_block(const SweepParams &P, const int b) {
     constexpr int G32 = LEAN >= 2 ? LEAN - 1 : 0;
