@@ -63,9 +63,8 @@ extern "C" {
 
 /* Precision of the overlap tests.  RP_PREC_FP64 evaluates every test in the reference's FP64 operation order.
  * RP_PREC_GUARDED_FP32 (no counterpart in the reference): the stencil scan of the default hard spherocylinder sweep
- * (eight wavefronts per cell, grouped moves; other launches and shapes keep FP64) takes squared centre distances in
- * FP32 from positions
- * relative to the active cell's centre, with rigorous bounds on their error; a pair whose FP32 value lies within that
+ * (eight wavefronts per cell, speculative moves; other launches and shapes keep FP64) takes squared centre distances in
+ * FP32 from positions relative to the active cell's centre, with rigorous bounds on their error; a pair whose FP32 value lies within that
  * bound of contact or of the interaction range is decided by the FP64 value, so every decision equals RP_PREC_FP64's.
  * Box, inverse, positions and the segment-distance stage stay FP64.  RP_PREC_GUARDED_FP32_VERIFY also evaluates every
  * pair in FP64 and records the largest FP32 error and any class that differs (rp_get_guard_stats). */
@@ -338,10 +337,10 @@ int rp_get_timing(rp_ctx *ctx, rp_timing *out);
 
 /* Launch-shape autotuner (no counterpart in the reference, whose domain decomposition has no launch shape): runs
  * cycles_per_shape cycles (no step adaptation) with each candidate sweep launch -- wavefronts per active cell and
- * the move schedule (0 plain, 1 planner/tester pipeline, 2 grouped moves) -- timing every sweep launch, and keeps
+ * the move schedule (0 plain, 1 planner/tester pipeline, 2 grouped or speculative moves) -- timing every sweep launch, and keeps
  * the fastest for the cycles that follow.  Every launch shape makes the same decisions, so the call is
  * rp_run_cycles(ctx, candidates x cycles_per_shape, 0, NULL) bit for bit, whatever shape it keeps.  Candidates: hard
- * spheres and spherocylinders all six tested shapes (the guarded FP32 precision only its grouped eight-wavefront
+ * spheres and spherocylinders all six tested shapes (the guarded FP32 precision only its eight-wavefront
  * launch), polyspheres 1, 2, 4, 8 or 16 wavefronts; soft and overlap-counting sweeps keep their shape.  out (nullable,
  * RP_AUTOTUNE_MAX entries) receives each candidate and its mean sweep time per cycle, *n_out their number and
  * *chosen (nullable) the index kept. */

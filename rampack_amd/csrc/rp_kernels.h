@@ -245,11 +245,12 @@ hipError_t launch_mlp_pairs(hipStream_t s, const SweepParams &sp, int M, uint64_
 int sweep_occupancy(int kind, int cap, int waves);
 // g32: 0 FP64 stencil scan; 1 guarded FP32 scan; 2 guarded FP32 scan that also evaluates every pair in FP64 and
 // records the largest FP32 error and any class mismatch (counters CNT_G32_*).  g32 > 0 needs eight wavefronts, the
-// grouped launch and a hard sphere or spherocylinder.
+// speculative launch and a hard spherocylinder.
 hipError_t launch_sweep(hipStream_t s, const SweepParams &sp, int waves, Timed t = {}, int g32 = 0);
 size_t sweep_lds_bytes(int kind, int cap, int waves, int g32 = 0, bool lean = false);
-// Whether a (non-fix) sweep of this launch shape runs the speculative kernel.
-int sweep_lean_cap();  // stencil entries it can stage at most
+// Whether a (non-fix) sweep of this launch shape runs a speculative kernel, and the stencil entries the spherocylinders'
+// can stage at most.
+int sweep_lean_cap();
 bool sweep_is_lean(const PairConsts &k, int waves, int pipelined, bool counting);
 // The kernel launch_sweep(sp, waves, g32) would run, as a key shared by the packings one batched launch may hold, or
 // -1 for the sweeps that run one packing per launch (soft, overlap counting, orientation fix, polyspheres, traced).
