@@ -2688,6 +2688,7 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
     int word = firstWord;
     for (int chunk = 0; chunk < moves; chunk += SPEC_MOVES) {
         const int cn = min(SPEC_MOVES, moves - chunk);
+        if (chunk > 0) __syncthreads();  // every wavefront has read the last chunk's final command
         if (wave == 0) {
             if (chunk > 0 && lane < cn) {
                 spec_proposal(P, L, lane, pbase + chunk + lane);

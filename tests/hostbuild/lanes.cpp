@@ -208,10 +208,12 @@ bool resolve_block(bool &finished) {
 }
 
 // Order in which wavefronts advance: all runnable lanes in lane order, then every wavefront's operations (the
-// default); or, with EMU_SCHED_SEED set, one wavefront at a time drawn at random among those that can advance, so
-// that wavefronts run ahead of each other between workgroup barriers by random amounts.
+// default); or, with EMU_SCHED_SEED set, one wavefront at a time among those that can advance: drawn at random (a
+// number), so that wavefronts run ahead of each other between workgroup barriers by random amounts, or always the first
+// ("lowest") or the last ("highest").
+enum SchedOrder { TOGETHER, RANDOM, LOWEST, HIGHEST };
 uint64_t schedState = 0;
-bool schedRandom = false;
+SchedOrder schedOrder = TOGETHER;
 
 uint64_t next_random() {
     schedState += 0x9E3779B97F4A7C15ull;
@@ -225,7 +227,7 @@ void run_block() {
     const std::size_t nt = nLanes;
     bool finished = false;
     while (!finished) {
-        if (!schedRandom) {
+        if (schedOrder == TOGETHER) {
             bool ran = false;
             for (std::size_t i = 0; i < nt; i++)
                 if (lanes[i].state == RUNNABLE) {
@@ -254,7 +256,8 @@ void run_block() {
             if (!resolve_block(finished)) deadlock("deadlock (no lane can proceed)");
             continue;
         }
-        const std::size_t w = cand[next_random() % (uint64_t)nc];
+        const std::size_t w = schedOrder == LOWEST ? cand[0] : schedOrder == HIGHEST ? cand[nc - 1]
+                                                             : cand[next_random() % (uint64_t)nc];
         bool ran = false;
         for (std::size_t i = w; i < std::min(nt, w + 64); i++)
             if (lanes[i].state == RUNNABLE) {
@@ -307,8 +310,8 @@ void run_grid(dim3 grid, dim3 block, std::size_t lds, const std::function<void()
     if (!seeded) {
         seeded = true;
         if (const char *sd = std::getenv("EMU_SCHED_SEED")) {
-            schedRandom = true;
-            schedState = std::strtoull(sd, nullptr, 10);
+            schedOrder = !std::strcmp(sd, "lowest") ? LOWEST : !std::strcmp(sd, "highest") ? HIGHEST : RANDOM;
+            if (schedOrder == RANDOM) schedState = std::strtoull(sd, nullptr, 10);
         }
     }
     body = &b;
