@@ -904,14 +904,20 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count_overlaps(Grid g, Partic
                                                                   unsigned long long *counters, int cap, int rot) {
     extern __shared__ double smem[];
     __shared__ int s_start[MAX_HALF + 1], s_base[MAX_HALF], s_ecode[MAX_HALF];
-    __shared__ int sFound;
+    __shared__ int sFound, sStop;
     __shared__ double sT[81];
     const int tid = threadIdx.x;
     const int cell = (int)((blockIdx.x + (unsigned)rot) % (unsigned)g.ncell);
     const int own0 = g.cellStart[cell];
     const int nOwn = g.cellStart[cell + 1] - own0;
     if (nOwn == 0) return;
-    if (earlyExit && overlap_found(counters)) return;
+    if (earlyExit) {
+        // One thread reads the flag for the workgroup: another workgroup may raise it between two wavefronts' reads, and
+        // wavefronts that stay alone would go on with a table in LDS that the others never filled.
+        if (tid == 0) sStop = overlap_found(counters) ? 1 : 0;
+        __syncthreads();
+        if (sStop) return;
+    }
     const int cx = cell % g.n[0], cy = (cell / g.n[0]) % g.n[1], cz = cell / (g.n[0] * g.n[1]);
     const int ncells = stencil_cells(g.reach, true);
     for (int i = tid; i < 81; i += COUNT_THREADS) sT[i] = g.T[i];
@@ -958,12 +964,14 @@ template <int KIND>
 __global__ __launch_bounds__(COUNT_THREADS) void k_count_items(Grid g, int n, Particles p, PairConsts k, int earlyExit,
                                                                unsigned long long *counters, int cap, int rot) {
     __shared__ double sT[81], sBeadR[RP_MAX_CENTRES];
+    __shared__ int sStop;
     const int tid = threadIdx.x;
-    if (earlyExit && overlap_found(counters)) return;
+    if (tid == 0) sStop = earlyExit && overlap_found(counters) ? 1 : 0;  // one decision per workgroup
     for (int i = tid; i < 81; i += COUNT_THREADS) sT[i] = g.T[i];
     if (KIND == 2)
         for (int c = tid; c < k.nc; c += COUNT_THREADS) sBeadR[c] = k.beads[4 * c + 3];
     __syncthreads();
+    if (sStop) return;
     // the items from those of cell `rot` on, then the ones before
     const int at = (int)blockIdx.x * (COUNT_THREADS / COUNT_LANES) + tid / COUNT_LANES, sub = tid % COUNT_LANES;
     const int ncells = stencil_cells(g.reach, true);

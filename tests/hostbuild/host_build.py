@@ -2,8 +2,9 @@
 rampack_amd/csrc compiled by g++ against the host stand-in of the HIP runtime (include/hip/hip_runtime.h), with
 AddressSanitizer.  Test infrastructure: nothing in the package loads it.
 
-The one textual change to the sources: a kernel's dynamic LDS declaration (`extern __shared__ T name[];`) becomes a
-pointer to the launch's LDS allocation, which has exactly the size the launch asks for.
+Two textual changes to the sources: a kernel's dynamic LDS declaration (`extern __shared__ T name[];`) becomes a
+pointer to the launch's LDS allocation, which has exactly the size the launch asks for, and every declaration of static
+`__shared__` variables is followed by calls that fill them when a workgroup first passes it.
 
     python tests/hostbuild/host_build.py [csrc_dir [library]]   # optional: another copy of rampack_amd/csrc, output path
 """
@@ -34,6 +35,11 @@ def host_kernel_source(src: str) -> str:
                       r"\1 *\2 = static_cast<\1 *>(emu::dyn_lds());", text)
     if n == 0:
         raise RuntimeError(f"{src}: no dynamic LDS declaration found")
+    def fill(m):
+        names = re.findall(r"(\w+)\s*(?:\[|,|;)", re.sub(r"\[[^\]]*\]", "[", m.group(0)))
+        return m.group(0) + "".join(f" emu::static_lds(&{n}, sizeof {n});" for n in names)
+
+    text = re.sub(r"__shared__\s+[^;()]*;", fill, text)
     out = os.path.join(OUT_DIR, "rp_kernels_host.cpp")
     with open(out, "w") as f:
         f.write(f'#line 1 "{src}"\n')

@@ -6,7 +6,9 @@
 // resolved once every live lane of the block has reached its next such point, over the lanes that reached the same
 // operation (the lanes a divergent branch leaves out do not take part, as with an execution mask).  Device memory is
 // host heap memory and every allocation, the dynamic LDS of each launch included, is exactly the size asked for, so
-// that AddressSanitizer reports any access outside it.
+// that AddressSanitizer reports any access outside it.  LDS, static variables included, holds a fill pattern when a
+// workgroup starts (EMU_LDS_FILL, a byte), and a flag that another workgroup of the launch may raise can change between
+// two wavefronts' reads of it (EMU_FLAG_ODDS).
 #pragma once
 
 #include <cfloat>
@@ -72,6 +74,8 @@ extern dim3 blockIdxV, blockDimV, gridDimV;
 
 unsigned lane_tid();
 void *dyn_lds();
+void static_lds(void *p, std::size_t n);  // follows every declaration of static __shared__ variables (host_build.py)
+uint64_t flag_load(const uint64_t *p);
 
 enum WaveKind { W_BALLOT, W_SHFL, W_SHFL_DOWN, W_SHFL_XOR, W_READLANE, W_READFIRST, W_BARRIER, W_SHFL_UP };
 uint64_t wave_op(int kind, uint64_t bits, int arg, int line);
@@ -165,6 +169,7 @@ inline unsigned __smid() { return 0; }
 #endif
 template <class T>
 inline T __hip_atomic_load(const T *p, int, int) {
+    if constexpr (sizeof(T) == 8) return (T)emu::flag_load(reinterpret_cast<const uint64_t *>(p));
     return *p;
 }
 template <class T, class U>

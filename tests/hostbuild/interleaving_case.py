@@ -4,6 +4,7 @@ per process, draws the order in which the wavefronts of a workgroup advance).
     python tests/hostbuild/interleaving_case.py LIB rods N_SIDE SPACING STEP SAMPLERS PRECISION CYCLES
     python tests/hostbuild/interleaving_case.py LIB chains BEADS N_SIDE SPACING STEP SAMPLERS CYCLES
     python tests/hostbuild/interleaving_case.py LIB nogrid N_SIDE SPACING STEP SAMPLERS CYCLES
+    python tests/hostbuild/interleaving_case.py LIB count KIND   # early-exit overlap counts; EMU_FLAG_ODDS raises the flag
 
 N_SIDE and SPACING are three numbers joined by commas.
 """
@@ -83,6 +84,24 @@ def nogrid(n_side, spacing, step, samplers, cycles):
     pk.close()
 
 
+def count(kind):
+    """Layers of particles with a gap between them, so that cells without any alternate with full ones, and one
+    overlapping pair: the early-exit count is 1 whichever workgroup finds it and whenever the others learn of it."""
+    if kind == "rods":
+        shape, (box, pos, rot) = SC, lattice.spherocylinder_lattice((16, 16, 4), (1.3, 1.3, 15.0))
+    elif kind == "spheres":
+        shape, (box, pos, rot) = ra.Shape("sphere", radius=0.5), lattice.hard_sphere_lattice(10, 0.3)
+    else:
+        from test_gpu_poly import chain_start
+        shape = ra.Shape("polysphere", centres=[[0, 0, -0.5], [0, 0, 0.5]], radii=[0.5, 0.5])
+        box, pos, rot = chain_start((9, 9, 6), (1.3, 1.3, 4.5))
+    pos[-1] = pos[-2] + [0.3, 0.0, 0.0]
+    pk = ra.GpuPacking(shape, box, pos, rot, seed=3)
+    for _ in range(40):
+        assert pk.count_total_overlaps(True) == 1
+    pk.close()
+
+
 if __name__ == "__main__":
-    {"rods": rods, "chains": chains, "nogrid": nogrid}[sys.argv[2]](*sys.argv[3:])
+    {"rods": rods, "chains": chains, "nogrid": nogrid, "count": count}[sys.argv[2]](*sys.argv[3:])
     print("case passed", flush=True)

@@ -213,6 +213,9 @@ bool resolve_block(bool &finished) {
 // ("lowest") or the last ("highest").
 enum SchedOrder { TOGETHER, RANDOM, LOWEST, HIGHEST };
 uint64_t schedState = 0;
+int ldsFill = 0xA5;
+uint64_t flagOdds = 0, flagSeen[16];
+std::vector<const void *> staticSeen;  // this workgroup's static LDS variables so far
 SchedOrder schedOrder = TOGETHER;
 
 uint64_t next_random() {
@@ -273,6 +276,26 @@ void run_block() {
 unsigned lane_tid() { return cur->tid; }
 void *dyn_lds() { return dynLds; }
 
+// The first lane of a workgroup to pass the declaration fills the variable: what LDS holds then is another kernel's.
+void static_lds(void *p, std::size_t n) {
+    for (const void *q : staticSeen)
+        if (q == p) return;
+    staticSeen.push_back(p);
+    std::memset(p, ldsFill, n);
+}
+
+// An atomic read of a 64-bit word at device scope.  With EMU_FLAG_ODDS = k, every k-th wavefront or so that reads a zero
+// finds it raised to one just then, as by a workgroup running elsewhere; a wavefront's lanes read the same value.
+uint64_t flag_load(const uint64_t *p) {
+    if (!flagOdds) return *p;
+    const unsigned w = cur->tid / 64;
+    if (cur->tid % 64 == 0) {
+        if (*p == 0 && next_random() % flagOdds == 0) *const_cast<uint64_t *>(p) = 1;
+        flagSeen[w] = *p;
+    }
+    return flagSeen[w];
+}
+
 uint64_t wave_op(int kind, uint64_t bits, int arg, int line) {
     Lane &l = *cur;
     l.state = AT_WAVE;
@@ -313,6 +336,8 @@ void run_grid(dim3 grid, dim3 block, std::size_t lds, const std::function<void()
             schedOrder = !std::strcmp(sd, "lowest") ? LOWEST : !std::strcmp(sd, "highest") ? HIGHEST : RANDOM;
             if (schedOrder == RANDOM) schedState = std::strtoull(sd, nullptr, 10);
         }
+        if (const char *f = std::getenv("EMU_LDS_FILL")) ldsFill = std::atoi(f);
+        if (const char *k = std::getenv("EMU_FLAG_ODDS")) flagOdds = std::strtoull(k, nullptr, 10);
     }
     body = &b;
     blockDimV = block;
@@ -324,7 +349,9 @@ void run_grid(dim3 grid, dim3 block, std::size_t lds, const std::function<void()
             for (unsigned bx = 0; bx < grid.x; bx++) {
                 blockIdxV = dim3(bx, by, bz);
                 // LDS starts with no defined contents: fill it with a pattern that makes stale reads visible
-                std::memset(dynLds, 0xA5, lds ? lds : 1);
+                std::memset(dynLds, ldsFill, lds ? lds : 1);
+                staticSeen.clear();
+                std::memset(flagSeen, 0, sizeof flagSeen);
                 for (std::size_t i = 0; i < nt; i++) {
                     lanes[i].tid = (unsigned)i;
                     start_lane(lanes[i]);

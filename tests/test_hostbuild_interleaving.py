@@ -1,7 +1,11 @@
-"""The speculative sweeps on the CPU build (tests/hostbuild) under different orders of the wavefronts between barriers:
-the lowest wavefront always first, the highest always first, and drawn orders.  A missing barrier shows as another
-trajectory than that of one wavefront making one move at a time.  Cells have more moves than a chunk holds, so that a
-chunk's end and the next one's start meet."""
+"""What the order of wavefronts can change, on the CPU build (tests/hostbuild).
+
+* The speculative sweeps under different orders of the wavefronts between barriers: the lowest wavefront always first, the
+  highest always first, and drawn orders.  A missing barrier shows as another trajectory than that of one wavefront making
+  one move at a time.  Cells have more moves than a chunk holds, so that a chunk's end and the next one's start meet.
+* Early-exit overlap counts whose flag another workgroup raises between two wavefronts' reads of it, with LDS as another
+  kernel may have left it: no access outside an allocation, and the same count.
+"""
 import os
 import subprocess
 import sys
@@ -51,3 +55,10 @@ def test_chains_follow_one_wavefront(host_lib, order):
 @pytest.mark.parametrize("order", ["lowest", "highest", "3"])
 def test_packings_without_a_grid_replay(host_lib, order):
     run_case(host_lib, "nogrid", "8,8,2", "1.6,1.6,6.6", 0.1, 1, 2, EMU_SCHED_SEED=order)
+
+
+@pytest.mark.parametrize("fill", ["1", "165"])
+@pytest.mark.parametrize("order", ["lowest", "highest", "3"])
+@pytest.mark.parametrize("kind", ["rods", "spheres", "beads"])
+def test_early_exit_flag_raised_between_two_wavefronts(host_lib, kind, order, fill):
+    run_case(host_lib, "count", kind, EMU_FLAG_ODDS="9", EMU_LDS_FILL=fill, EMU_SCHED_SEED=order)
