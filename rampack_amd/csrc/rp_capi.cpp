@@ -1166,10 +1166,11 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
     if (waves == 16 && (c->k.kind != RP_SHAPE_POLYSPHERE || c->k.soft || c->counting)) waves = 8;
     // eight wavefronts only for the hard sweeps
     if (waves == 8 && (c->k.soft || c->counting)) waves = 4;
-    // the eight-wavefront kernels that make one move at a time write no per-sampler acceptance flags (no registers to spare
-    // for them); the speculative sweeps do
-    if (waves >= 8 && ms.n > 1 && !hardRods && c->k.kind != RP_SHAPE_POLYSPHERE) waves = 4;
-    sp.pipelined = c->pipelined >= 0 ? c->pipelined : (waves >= 8 ? 2 : 1);
+    // the kernels of eight wavefronts and more that are not speculative write no per-sampler acceptance flags (no registers
+    // to spare for them): judged by the kernel that will run, with a pinned schedule (rp_autotune) as without
+    const auto schedule = [&](int w) { return c->pipelined >= 0 ? c->pipelined : (w >= 8 ? 2 : 1); };
+    if (waves >= 8 && ms.n > 1 && !sweep_is_lean(c->k, waves, schedule(waves), c->counting)) waves = 4;
+    sp.pipelined = schedule(waves);
     // guarded FP32 stencil scan: the default launch of hard spherocylinders (eight wavefronts, speculative moves); the
     // all-pairs path (no grid) tests in FP64
     const int g32 = c->precision != RP_PREC_FP64 && waves == 8 && sp.pipelined == 2 && !c->k.soft && !c->counting &&
