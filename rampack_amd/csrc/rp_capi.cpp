@@ -1151,11 +1151,20 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
     cap = (cap + 63) / 64 * 64;
     int waves = c->sweepWaves;
     // Eight wavefronts for dense stencils, else fewer.  Hard spherocylinders take the eight of the speculative sweep from
-    // 180 particles per stencil on (200 cycles of 16 000 rods at 220: 48.6 ms against 53.6 on one wavefront, at 300 49.2
-    // against 75.5; 3 456 rods at 155: 45.1 against 43.7).  Two wavefronts with a planner, which ran at 128 to 384 before,
-    // faulted the GPU on layered packings with partly empty cells, and the cause is not found.
+    // 180 particles per stencil on while all workgroups of a colour pass run at once (two per compute unit, 512): 10 976
+    // rods at 212, 175 workgroups, 60 cycles: 14.7 ms, 16.1 on one or two wavefronts; 4 608 at 156, 13.4 against 13.2.
+    // Beyond, where lanes left idle cost throughput, from 240 (several samplers, whose chunks hold more accepted moves:
+    // 280): 36 000 rods at 201, 605 workgroups, 18.2 ms against 16.3 on two, with two samplers 34.6 against 25.9; at 243
+    // 15.8 against 18.6 and 28.7 against 30.6; 291 600 at 264, 63.8 against 84.3 and 166 against 159 (two samplers, short
+    // steps).  Between, two wavefronts with a planner from 180 on, and from 128 on over 1024 workgroups (291 600 rods at
+    // 160, 72.2 ms, 75.1 on one wavefront; 28 800 at 169, 576 workgroups, 14.9 against 14.4).
     const bool hardRods = c->k.kind == RP_SHAPE_SPHEROCYLINDER && !c->k.soft && !c->counting && c->pipelined < 0;
-    if (waves <= 0) waves = hardRods ? (expect > 180 ? 8 : 1) : (expect > 384 ? 8 : (expect > 128 ? 2 : 1));
+    if (waves <= 0 && hardRods) {
+        const long long blocks = (long long)sp.na[0] * sp.na[1] * sp.na[2];
+        const double eight = blocks <= 512 ? 180 : (ms.n == 1 ? 240 : 280);
+        waves = expect > eight ? 8 : (expect > (blocks <= 1024 ? 180 : 128) ? 2 : 1);
+    }
+    if (waves <= 0) waves = expect > 384 ? 8 : (expect > 128 ? 2 : 1);
     // hard polyspheres: the speculative sweep on eight or sixteen wavefronts once a stencil holds some 200 particles, one
     // move at a time below that (10 cycles on 5-bead chains, stencils of 270: 14.8 ms against 17.2 with two wavefronts one
     // at a time; 3-bead chains, 130: 9.2 on four wavefronts against 7.7; 7-bead chains, 650: sixteen 16.0, eight 16.3)

@@ -4,6 +4,7 @@ for), and its decisions replay through the oracle."""
 import pytest
 
 import rampack_amd as ra
+from rampack_amd import lattice
 from test_gpu_replay import SC, check_record, rod_start
 
 pytestmark = pytest.mark.gpu
@@ -36,4 +37,24 @@ def test_autotuned_guarded_sweep_of_two_samplers_stays_guarded():
     before = pk.guard_stats()["pairs"]
     pk.run_cycles(2)
     assert pk.timing()["sweep_waves"] == 8 and pk.guard_stats()["pairs"] > before > 0
+    pk.close()
+
+
+@pytest.mark.parametrize("n_side, spacing, samplers, waves", [
+    ((28, 28, 6), (2.2, 2.2, 6.6), 1, 8),    # stencils of 212, 75 workgroups per colour: the chip is not full
+    ((60, 60, 10), (2.2, 2.2, 6.6), 1, 2),   # 201, 605 workgroups
+    ((60, 60, 10), (2.2, 2.2, 6.6), 2, 2),
+    ((60, 60, 10), (2.6, 2.6, 7.0), 1, 1),   # 144, 845 workgroups
+    ((60, 60, 10), (1.8, 1.8, 6.6), 2, 8),   # 300, 405 workgroups
+    ((86, 86, 24), (2.4, 2.4, 6.4), 1, 2),   # about 160, over 1024 workgroups
+])
+def test_thin_stencils_of_rods(n_side, spacing, samplers, waves):
+    box, pos, rot = lattice.spherocylinder_lattice(n_side, spacing)
+    pk = ra.GpuPacking(SC, box, pos, rot, seed=7)
+    pk.set_environment(1.0, 0.5, 0.2, None, box_move=("log", 0.001))
+    if samplers > 1:
+        pk.set_move_samplers([("translation", 0.2), ("rotation", 0.2)])
+    pk.run_cycles(3)
+    assert pk.timing()["sweep_waves"] == waves
+    check_record(SC, pk.record_sweep(), rejections=False)
     pk.close()
