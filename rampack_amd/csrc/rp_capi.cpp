@@ -1200,7 +1200,6 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
     const double perEntry = (double)(sweep_lds_bytes(c->k.kind, 1024, waves, g32, lean) - fixed) / 1024.0;
     const int maxCap = poly ? 64 : (int)((double)(c->ldsLimit - fixed) / perEntry) / 64 * 64;
     sp.cap = std::max(64, std::min(cap, maxCap));
-    if (lean) sp.cap = std::min(sp.cap, sweep_lean_cap());
     // workgroups that read their stencil from HBM so far (hCounters as of the last read)
     if (!c->pairCapOff && c->blocksAtRead >= 10000 && c->hCounters[CNT_UNSTAGED_BLOCKS] * 100 > c->blocksAtRead)
         c->pairCapOff = true;

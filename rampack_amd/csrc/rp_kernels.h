@@ -248,9 +248,7 @@ int sweep_occupancy(int kind, int cap, int waves);
 // speculative launch and a hard spherocylinder.
 hipError_t launch_sweep(hipStream_t s, const SweepParams &sp, int waves, Timed t = {}, int g32 = 0);
 size_t sweep_lds_bytes(int kind, int cap, int waves, int g32 = 0, bool lean = false);
-// Whether a (non-fix) sweep of this launch shape runs a speculative kernel, and the stencil entries the spherocylinders'
-// can stage at most.
-int sweep_lean_cap();
+// Whether a (non-fix) sweep of this launch shape runs a speculative kernel.
 bool sweep_is_lean(const PairConsts &k, int waves, int pipelined, bool counting);
 // The kernel launch_sweep(sp, waves, g32) would run, as a key shared by the packings one batched launch may hold, or
 // -1 for the sweeps that run one packing per launch (soft, overlap counting, orientation fix, polyspheres, traced).

@@ -2321,7 +2321,7 @@ constexpr double SPEC_FAR = 1e17;  // position of a trial pose that is not to be
 constexpr int SPEC_QNEAR = WAVE + SPEC_UNIT * WAVE;  // pairs within the range: drained to below 64 before every unit
 constexpr int SPEC_QSEG = 2 * WAVE;                   // pairs for the segment test: drained to below 64 after every drain
 constexpr int SPEC_QUEUE = SPEC_QNEAR + SPEC_QSEG;    // entries (candidate << 5 | move, 16 bits) per wavefront
-constexpr int SPEC_CAP = 2048;                        // candidates an entry can name
+constexpr int SPEC_PAGE = 2048;                       // candidates an entry can name: the queues are emptied between pages
 constexpr int SPEC_INTS = SPEC_MOVES + 2 * SPEC_MOVES + 6;  // plan words, ownHit, hitOut, command, moved 2, spare 2
 
 struct SpecLds {
@@ -2468,12 +2468,12 @@ __device__ __forceinline__ void spec_hit(const SpecLds &L, int j, int m, int nOw
 
 // The exact segment tests of at most 64 queued pairs, one per lane; pairs of moves already dead skip.
 __device__ __forceinline__ void spec_segments(const SpecConsts &K, const Stencil &S, const SpecLds &L, bool translated,
-                                              const uint16_t *entries, int n, int nOwn, unsigned dead) {
+                                              const uint16_t *entries, int n, int page, int nOwn, unsigned dead) {
     constexpr int M = SPEC_MOVES;
     const int lane = threadIdx.x & (WAVE - 1);
     __builtin_amdgcn_wave_barrier();  // the queue was written by other lanes of this wavefront
     if (lane < n) {
-        const int e = entries[lane], j = e >> 5, m = e & (M - 1);
+        const int e = entries[lane], j = page + (e >> 5), m = e & (M - 1);
         if (!((dead >> m) & 1)) {
             V3 c2 = v3(S.x[j], S.y[j], S.z[j]);
             if (!translated) {
@@ -2495,8 +2495,8 @@ __device__ __forceinline__ void spec_segments(const SpecConsts &K, const Stencil
 // The near tests of at most 64 queued pairs, one per lane: in contact by the centre distance (a hit), beyond the range,
 // or separated (dropped), else queued for the segment test.  segQueued: entries of the second queue (updated).
 __device__ __forceinline__ void spec_near(const SpecConsts &K, const Stencil &S, const SpecLds &L, bool translated,
-                                          const uint16_t *entries, int n, uint16_t *segQueue, int &segQueued, int nOwn,
-                                          unsigned dead) {
+                                          const uint16_t *entries, int n, int page, uint16_t *segQueue, int &segQueued,
+                                          int nOwn, unsigned dead) {
     constexpr int M = SPEC_MOVES;
     const int lane = threadIdx.x & (WAVE - 1);
     __builtin_amdgcn_wave_barrier();  // the queue was written by other lanes of this wavefront
@@ -2504,7 +2504,7 @@ __device__ __forceinline__ void spec_near(const SpecConsts &K, const Stencil &S,
     int e = 0;
     if (lane < n) {
         e = entries[lane];
-        const int j = e >> 5, m = e & (M - 1);
+        const int j = page + (e >> 5), m = e & (M - 1);
         if (!((dead >> m) & 1)) {
             const int w = L.word[m];
             V3 p2 = v3(S.x[j], S.y[j], S.z[j]);
@@ -2587,15 +2587,16 @@ __device__ __forceinline__ void spec_unit(const SpecConsts &K, const SpecLds &L,
         if (within)
             nearQ[nearN + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(am >> 32),
                                                          __builtin_amdgcn_mbcnt_lo((unsigned)am, 0u))] =
-                (uint16_t)((j << 5) | m[k]);
+                (uint16_t)((j << 5) | m[k]);  // (j within its page)
         nearN += __popcll(am);
     }
 }
 
 // Scans the stencil for the moves of `active` (all inside the cell): the first scan of a chunk (whole = true: every
 // move that is not in `active` has its trial position SPEC_FAR away) in units of consecutive moves, a rescan in
-// units of up to four of its moves.
-template <int KIND, int WAVES, int G32>
+// units of up to four of its moves.  PAGED: the stencil has more candidates than a queue entry names (a path of its own:
+// the page in every index costs 1 % of a sweep of 1e5 rods).
+template <int KIND, int WAVES, int G32, bool PAGED>
 __device__ __forceinline__ void spec_scan(const SpecConsts &K, const Stencil &S, const SpecLds &L, bool translated,
                                           int nOwn, int total, unsigned active, bool whole, SpecStats &st) {
     static_assert(KIND == 1, "the queues serve spherocylinders");
@@ -2607,7 +2608,7 @@ __device__ __forceinline__ void spec_scan(const SpecConsts &K, const Stencil &S,
     const int nslots = (total + WAVE - 1) / WAVE;
     const unsigned skipDead = G32 == 2 ? 0u : ~0u;  // verify mode evaluates every pair
     unsigned dead = lds_mask(L.hitOut) & skipDead;
-    int s = wave, grp = 0;
+    int s = wave, grp = 0, page = 0;  // page: the first candidate of the queued entries' page
     unsigned rest = active;  // rescans: the moves of this and the later groups
     int ngroups = whole ? (SPEC_MOVES - __builtin_clz(active) + UNIT - 1) / UNIT : (__popc(active) + 3) / 4;
     for (;;) {
@@ -2617,7 +2618,18 @@ __device__ __forceinline__ void spec_scan(const SpecConsts &K, const Stencil &S,
             if (!whole)
                 for (int k = 0; k < 4; k++) rest &= rest - 1;  // (stays 0 once it is)
         }
-        if (grp >= ngroups) break;
+        const bool end = grp >= ngroups;
+        if (end || (PAGED && (s * WAVE & -SPEC_PAGE) != page)) {
+            if (nearN > 0) spec_near(K, S, L, translated, nearQ, nearN, page, segQ, segN, nOwn, dead);
+            nearN = 0;
+            while (segN > 0) {
+                const int n = min(segN, WAVE);
+                segN -= n;
+                spec_segments(K, S, L, translated, segQ + segN, n, page, nOwn, dead);
+            }
+            if (end) break;
+            page = PAGED ? s * WAVE & -SPEC_PAGE : 0;
+        }
         const int j = s * WAVE + lane;
         const bool valid = j < total;
         const int jj = valid ? j : 0;
@@ -2653,20 +2665,14 @@ __device__ __forceinline__ void spec_scan(const SpecConsts &K, const Stencil &S,
         }
         while (nearN >= WAVE) {
             nearN -= WAVE;
-            spec_near(K, S, L, translated, nearQ + nearN, WAVE, segQ, segN, nOwn, dead);
+            spec_near(K, S, L, translated, nearQ + nearN, WAVE, page, segQ, segN, nOwn, dead);
             if (segN >= WAVE) {
                 segN -= WAVE;
-                spec_segments(K, S, L, translated, segQ + segN, WAVE, nOwn, dead);
+                spec_segments(K, S, L, translated, segQ + segN, WAVE, page, nOwn, dead);
                 dead |= lds_mask(L.hitOut) & skipDead;
             }
         }
         s += WAVES;
-    }
-    if (nearN > 0) spec_near(K, S, L, translated, nearQ, nearN, segQ, segN, nOwn, dead);
-    while (segN > 0) {
-        const int n = min(segN, WAVE);
-        segN -= n;
-        spec_segments(K, S, L, translated, segQ + segN, n, nOwn, dead);
     }
 }
 
@@ -2729,7 +2735,8 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
             const unsigned cmd = lds_mask(L.cmd);
             if (!cmd) break;
             const unsigned long long tc0 = clk ? wall_clock64() : 0;
-            spec_scan<KIND, WAVES, G32>(K, S, L, translated, nOwn, total, cmd, round == 0, st);
+            if (total <= SPEC_PAGE) spec_scan<KIND, WAVES, G32, false>(K, S, L, translated, nOwn, total, cmd, round == 0, st);
+            else spec_scan<KIND, WAVES, G32, true>(K, S, L, translated, nOwn, total, cmd, round == 0, st);
             __syncthreads();  // every hit of this scan is in LDS
             const unsigned long long tc1 = clk ? wall_clock64() : 0;
             if (clk) {
@@ -4555,8 +4562,6 @@ hipError_t launch_count_allpairs(hipStream_t s, const Grid &g, int n, Particles 
         return hipErrorInvalidValue;
     return hipGetLastError();
 }
-
-int sweep_lean_cap() { return SPEC_CAP; }
 
 bool sweep_is_lean(const PairConsts &k, int waves, int pipelined, bool counting) {
     return !k.soft && !counting && ((k.kind == 2 && waves >= 4) || (waves == 8 && pipelined == 2 && k.kind == 1));

@@ -1,6 +1,7 @@
 """A launch shape pinned by the autotuner or the environment runs the kernel that it names, with several move samplers as
 with one: eight wavefronts with schedule 2 on hard spherocylinders are the speculative sweep (guarded FP32 where asked
 for), and its decisions replay through the oracle."""
+import numpy as np
 import pytest
 
 import rampack_amd as ra
@@ -58,3 +59,23 @@ def test_thin_stencils_of_rods(n_side, spacing, samplers, waves):
     assert pk.timing()["sweep_waves"] == waves
     check_record(SC, pk.record_sweep(), rejections=False)
     pk.close()
+
+
+def test_stencils_of_over_2048_particles_stay_in_lds(monkeypatch):
+    """Layered rods of L/D = 10 in stencils of about 1 850 and up to 2 300 particles (the queue entries of the scan name
+    2048): the same cells as on one wavefront read their stencil from memory, and the trajectory is the same."""
+    shape = ra.Shape("spherocylinder", radius=0.5, length=10.0)
+    start = lattice.spherocylinder_lattice((46, 46, 7), (1.45, 1.45, 11.6))
+    runs = []
+    for waves in (None, "1"):
+        if waves:
+            monkeypatch.setenv("RAMPACK_SWEEP_WAVES", waves)
+        pk = ra.GpuPacking(shape, *start, seed=19)
+        pk.set_environment(1.0, 0.5, 0.05, None, box_move=None)
+        c = pk.run_cycles(10)
+        assert pk.timing()["sweep_waves"] == int(waves or 8) and pk.timing()["sweep_cap"] > 2048
+        runs.append((pk.download(), c["unstaged_blocks"]))
+        pk.close()
+    (s0, u0), (s1, u1) = runs
+    assert u0 == u1 > 0
+    assert all(np.array_equal(a, b) for a, b in zip(s0, s1))
