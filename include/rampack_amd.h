@@ -64,8 +64,9 @@ extern "C" {
 /* Precision of the overlap tests.  RP_PREC_FP64 evaluates every test in the reference's FP64 operation order.
  * RP_PREC_GUARDED_FP32 (no counterpart in the reference): the stencil scan of the default hard spherocylinder sweep
  * (eight wavefronts per cell, speculative moves; other launches and shapes keep FP64) takes squared centre distances in
- * FP32 from positions relative to the active cell's centre, with rigorous bounds on their error; a pair whose FP32 value lies within that
- * bound of contact or of the interaction range is decided by the FP64 value, so every decision equals RP_PREC_FP64's.
+ * FP32 from positions relative to the active cell's centre, with rigorous bounds on their error, and drops the pairs
+ * that are beyond the interaction range by more than the bound; every other pair is classified by its FP64 distance, so
+ * every decision equals RP_PREC_FP64's.
  * Box, inverse, positions and the segment-distance stage stay FP64.  RP_PREC_GUARDED_FP32_VERIFY also evaluates every
  * pair in FP64 and records the largest FP32 error and any class that differs (rp_get_guard_stats). */
 #define RP_PREC_FP64 0
@@ -393,7 +394,9 @@ int rp_pair_decisions_guarded_noalloc(const rp_shape_desc *shape, size_t n, cons
                                       uint8_t *d_decisions, uint8_t *d_codes, rp_guard_stats *stats);
 
 /* Precision of a context's sweeps (RP_PREC_*, as rp_create's argument), and the guarded sweep's statistics since the
- * context was created: pairs classified in FP32, fp64_fallback = pairs inside a guard band, and in verify mode
+ * context was created: pairs = the candidates of every move that stays in its cell, the moved particle itself left out;
+ * fp64_fallback = pairs that the scan found inside a guard band, which FP32 alone cannot classify (a move already rejected
+ * is not scanned on, except in verify mode); and in verify mode
  * mismatches (0) and max_err_centre (largest |FP32 - FP64| squared centre distance); the segment fields stay 0 (the
  * segment stage is FP64). */
 int rp_set_precision(rp_ctx *ctx, int precision);

@@ -85,9 +85,10 @@ struct SweepParams {
     unsigned long long *trace;   // optional per-workgroup record of one launch: start and end wall clock,
                                  // own | stencil << 16 | cell << 32, compute-unit id; nullptr when not tracing
     // Guarded FP32 stencil scan of the speculative sweep (G32 = 1 or 2): candidate positions relative to the
-    // active cell's centre in FP32, squared centre distances in FP32, and the FP64 value only for pairs the FP32 value
-    // cannot place on one side of a threshold.  g32Lim[s] = {contact2 lower, contact2 upper, range2 lower,
-    // range2 upper} bounds of the FP32 guard bands, s = 0 for cells whose stencil was staged translated (no wrapped
+    // active cell's centre in FP32 and squared centre distances in FP32, which drop the pairs certainly beyond the range;
+    // every pair below the upper end of the range's guard band is classified by its FP64 distance.  g32Lim[s] = {contact2
+    // lower, contact2 upper, range2 lower, range2 upper} bounds of the FP32 guard bands (those around contact serve the
+    // statistics), s = 0 for cells whose stencil was staged translated (no wrapped
     // particle), s = 1 otherwise (positions and image translations up to a box length from the centre).
     float g32Lim[2][4];
     double skip2;        // speculative sweep: a squared distance bound above which segments certainly do not touch
@@ -126,8 +127,8 @@ enum Counter : int {
     CNT_TYPE_ATT = 8,       // per move sampler (RP_MAX_MOVE_SAMPLERS entries): attempted moves
     CNT_TYPE_ACC = 12,      // per move sampler: accepted moves
     CNT_STAGE_OVERFLOW = 16,  // cells of an overlap count or energy sum too full to stage (cleared before each launch)
-    CNT_G32_PAIRS = 17,       // guarded FP32 sweep: (candidate, move) pairs classified from FP32 distances
-    CNT_G32_GUARD = 18,       // of those, pairs inside a guard band, decided by the FP64 distance
+    CNT_G32_PAIRS = 17,       // guarded FP32 sweep: (candidate, move) pairs, once per move that stays in its cell
+    CNT_G32_GUARD = 18,       // pairs the scan found inside a guard band, which FP32 alone cannot classify
     CNT_G32_MAXERR = 19,      // verify mode: largest |FP32 - FP64| squared centre distance (float bits)
     CNT_G32_MISMATCH = 20,    // verify mode: pairs whose guarded class differs from the FP64 class (0)
     CNT_SCAN_HINT = 21,       // a cell in which the last overlap count found an overlap

@@ -2373,10 +2373,9 @@ struct SpecConsts {
     int cap;
 };
 
-// Statistics of the guarded FP32 scan, per lane (pairs: per wavefront).
+// Statistics of the guarded FP32 scan, per lane.
 struct SpecStats {
     unsigned guard = 0, mismatch = 0;
-    unsigned long long pairs = 0;
     float err = 0.f;
 };
 
@@ -2573,8 +2572,10 @@ __device__ __forceinline__ void spec_unit(const SpecConsts &K, const SpecLds &L,
             // band, and the near stage classifies what it keeps from the FP64 distance
             const float x = d2f[k];
             within = x < K.lim[3];
-            if (within && ((x >= K.lim[0] && x < K.lim[1]) || x >= K.lim[2])) st.guard++;
-            if (G32 == 2 && lane < nvalid && d2[k] < 1e30) {
+            // (the moved particle itself is left out in verify mode only: a displacement rarely falls into a band)
+            const bool other = G32 != 2 || j != L.word[m[k]] >> 8;
+            if (within && ((x >= K.lim[0] && x < K.lim[1]) || x >= K.lim[2]) && other) st.guard++;
+            if (G32 == 2 && lane < nvalid && d2[k] < 1e30 && other) {
                 st.err = fmaxf(st.err, (float)fabs((double)x - d2[k]));
                 const bool c64 = d2[k] < K.contact2, w64 = d2[k] < K.range2;
                 if ((x < K.lim[0] && !c64) || (x >= K.lim[1] && c64) || (x < K.lim[2] && !w64) || (x >= K.lim[3] && w64))
@@ -2651,7 +2652,6 @@ __device__ __forceinline__ void spec_scan(const SpecConsts &K, const Stencil &S,
                 for (int k = 0; k < UNIT; k++) m[k] = UNIT * grp + k;
                 if (translated) spec_unit<UNIT, true, G32>(K, L, p2, fj, code, j, nvalid, m, nearQ, nearN, st);
                 else spec_unit<UNIT, false, G32>(K, L, p2, fj, code, j, nvalid, m, nearQ, nearN, st);
-                if (G32) st.pairs += (unsigned)(nvalid * __popc(todo));
             }
         } else {
             // one unit per move (stale moves are few)
@@ -2660,7 +2660,6 @@ __device__ __forceinline__ void spec_scan(const SpecConsts &K, const Stencil &S,
                 const int m[1] = {__builtin_ctz(r)};
                 if (translated) spec_unit<1, true, G32>(K, L, p2, fj, code, j, nvalid, m, nearQ, nearN, st);
                 else spec_unit<1, false, G32>(K, L, p2, fj, code, j, nvalid, m, nearQ, nearN, st);
-                if (G32) st.pairs += (unsigned)nvalid;
             }
         }
         while (nearN >= WAVE) {
@@ -2684,7 +2683,6 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
     const int tid = threadIdx.x;
     const int lane = tid & (WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    __shared__ unsigned long long sPairs;
     const int moves = P.moves > 0 ? P.moves : nOwn * P.mult;
     const int pbase = P.moves > 0 ? cell * P.moves : own0 * P.mult;
     unsigned long long accepted = 0, leftCell = 0, tests = 0, moved = 0;
@@ -2698,7 +2696,6 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
     if (G32)
         for (int i = 0; i < 4; i++) K.lim[i] = P.g32Lim[translated ? 0 : 1][i];
     unsigned long long tScan = 0, tRescan = 0, tDecide = 0, nRescans = 0;  // phase timers (clk)
-    if (G32 && tid == 0) sPairs = 0;
     int word = firstWord;
     for (int chunk = 0; chunk < moves; chunk += SPEC_MOVES) {
         const int cn = min(SPEC_MOVES, moves - chunk);
@@ -2877,15 +2874,15 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
             st.err = fmaxf(st.err, __shfl_xor(st.err, off));
         }
         if (lane == 0) {
-            atomicAdd(&sPairs, st.pairs);
             if (st.guard) atomicAdd(&P.counters[CNT_G32_GUARD], (unsigned long long)st.guard);
             if (G32 == 2) {
                 if (st.mismatch) atomicAdd(&P.counters[CNT_G32_MISMATCH], (unsigned long long)st.mismatch);
                 atomicMax(&P.counters[CNT_G32_MAXERR], (unsigned long long)__float_as_uint(st.err));
             }
         }
-        __syncthreads();
-        if (tid == 0) P.slots[(size_t)cell * SLOT_WORDS + SLOT_G32_PAIRS] = sPairs;
+        // every candidate but the moved particle itself, once per move that stays in its cell
+        if (tid == 0)
+            P.slots[(size_t)cell * SLOT_WORDS + SLOT_G32_PAIRS] = tests - ((unsigned long long)moves - leftCell);
     }
 }
 
