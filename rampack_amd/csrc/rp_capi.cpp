@@ -52,14 +52,32 @@ struct HostBox {
     }
 };
 
-// Packing::isBoxUpscaled (Packing.cpp:1155-1176)
-bool isBoxUpscaled(const HostBox &o, const HostBox &nb) {
-    const double EPS = 100 * 2.220446049250313e-16;
+// Whether disjoint convex particles certainly stay disjoint when the box goes from o to nb, so that no overlap scan is
+// needed: every side grows by one and the same factor (each pair's centre difference then grows along itself), or, for
+// spheres in a box with right angles, every side by its own (no centre distance shrinks).  Packing::isBoxUpscaled
+// (Packing.cpp:1155-1176) asks only for sides that grow and turn by less than 2e-14 in cos^2: a side of 200 may then move
+// by 3e-5 across itself, and unequal factors can push inclined rods together, so a legal packing could end with overlaps.
+bool cannotOverlap(const HostBox &o, const HostBox &nb, bool spheres) {
+    const double EPS = 2.220446049250313e-16;
+    double f[3], largest = 0;
     for (int i = 0; i < 3; i++) {
-        V3 os = o.side(i), ns = nb.side(i);
-        double d = dot(os, ns), n2o = dot(os, os), n2n = dot(ns, ns);
-        if (std::fabs(d * d / n2o / n2n - 1) > EPS) return false;
-        if (d * d / n2o / n2o < 1 + EPS) return false;
+        const V3 os = o.side(i), ns = nb.side(i);
+        f[i] = dot(os, ns) / dot(os, os);
+        if (!(f[i] >= 1 + 100 * EPS)) return false;
+    }
+    for (int e = 0; e < 9; e++) largest = std::max(largest, std::fabs(nb.dims[e]));
+    // the sides' elements within a few roundings of the scaled ones
+    auto scaled = [&](double f0, double f1, double f2) {
+        const double by[3] = {f0, f1, f2};
+        for (int e = 0; e < 9; e++)
+            if (!(std::fabs(nb.dims[e] - by[e % 3] * o.dims[e]) <= 8 * EPS * largest)) return false;
+        return true;
+    };
+    if (scaled(f[0], f[0], f[0])) return true;
+    if (!spheres || !scaled(f[0], f[1], f[2])) return false;
+    for (int i = 0; i < 3; i++) {
+        const V3 a = o.side(i), c = o.side((i + 1) % 3);
+        if (std::fabs(dot(a, c)) > 8 * EPS * std::sqrt(dot(a, a) * dot(c, c))) return false;
     }
     return true;
 }
@@ -786,7 +804,7 @@ int softBoxMove(rp_ctx *c, const HostBox &nb, double exponent, double u, const d
     r = rebuild(c, g, 1, c->box.inv);
     if (r) return r;
     c->boxScans++;
-    if (c->k.hardCore && !isBoxUpscaled(c->box, nb)) {
+    if (c->k.hardCore && !cannotOverlap(c->box, nb, c->k.kind == RP_SHAPE_SPHERE)) {
         // the compound's hard part: an overlap makes dE infinite (Packing.cpp:199-204); the compound is convex
         // (CompoundInteraction.cpp:25-31)
         uint64_t found = 0;
@@ -929,8 +947,7 @@ int hardBoxMove(rp_ctx *c, const HostBox &nb, double exponent, double u, const d
     // spheres and spherocylinders are convex; polyspheres are not (PolysphereTraits.h:133) and are always scanned,
     // bead by bead on the rescaled particles
     const bool poly = c->k.kind == RP_SHAPE_POLYSPHERE;
-    bool cannotOverlap = !poly && isBoxUpscaled(c->box, nb);
-    if (!cannotOverlap) {
+    if (poly || !cannotOverlap(c->box, nb, c->k.kind == RP_SHAPE_SPHERE)) {
         uint64_t found = 0;
         c->boxScans++;
         if (defer && !poly) {
@@ -2441,7 +2458,7 @@ int rp_try_scaling(rp_ctx *c, const double new_box[9], double *dE) {
             r = countBeads(c, c->alt.p, nb, 1, found);
             if (r) return r;
             if (found) result = INF;
-        } else if (!isBoxUpscaled(c->box, nb)) {  // spheres and spherocylinders are convex
+        } else if (!cannotOverlap(c->box, nb, c->k.kind == RP_SHAPE_SPHERE)) {  // spheres and spherocylinders are convex
             uint64_t found = 0;
             r = scanOverlaps(c, g, 1, found);
             if (r) return r;
