@@ -123,6 +123,8 @@ struct rp_ctx {
     unsigned long long *dCounters = nullptr;
     unsigned long long *dPhases = nullptr;  // sweep phase timers (RAMPACK_SWEEP_PHASES=1)
     int device = 0;                         // the HIP device the context was created on
+    int lastG32 = 0;                        // the last sweep's kernel, for the phase timers' report
+    bool lastLean = false;
     int sweepTuning = 0;                    // grouped sweep wave priorities (RAMPACK_SWEEP_TUNING)
     std::string tracePath;                  // per-workgroup trace of one sweep launch (RAMPACK_SWEEP_TRACE)
     uint64_t traceLaunch = 0, sweepLaunches = 0;
@@ -1251,6 +1253,8 @@ int planSweep(rp_ctx *c, bool logDecisions, SweepPlan &pl) {
     c->tstats.sweep_cap = (uint64_t)sp.cap;
     c->tstats.sweep_waves = (uint64_t)waves;
     c->tstats.sweep_period = (uint64_t)g.period;
+    c->lastG32 = g32;
+    c->lastLean = lean;
     return RP_OK;
 }
 
@@ -2231,7 +2235,8 @@ void rp_destroy(rp_ctx *c) {
                          ph[RP_PHASE_MOVES] / b / perUs, ph[RP_PHASE_WRITE] / b / perUs,
                          (unsigned long long)ph[RP_PHASE_BLOCKS], ph[RP_PHASE_LAST] / perUs, khz,
                          sweep_occupancy(c->shape.kind, c->tstats.sweep_cap ? (int)c->tstats.sweep_cap : 64,
-                                         c->tstats.sweep_waves ? (int)c->tstats.sweep_waves : 4));
+                                         c->tstats.sweep_waves ? (int)c->tstats.sweep_waves : 4, c->lastG32,
+                                         c->lastLean));
             if (ph[RP_PHASE_GROUPS] && ph[RP_PHASE_TOP] == 0) {
                 std::fprintf(stderr,
                              "speculative sweep per workgroup (us): first scan %.2f, rescans %.2f, decisions %.2f; %.2f "

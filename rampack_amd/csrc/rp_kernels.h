@@ -243,7 +243,7 @@ hipError_t launch_mlp_pairs(hipStream_t s, const SweepParams &sp, int M, uint64_
                             int *meta);
 
 // Workgroups of the sweep kernel one compute unit can hold at this LDS size (occupancy API).
-int sweep_occupancy(int kind, int cap, int waves);
+int sweep_occupancy(int kind, int cap, int waves, int g32, bool lean);
 // g32: 0 FP64 stencil scan; 1 guarded FP32 scan; 2 guarded FP32 scan that also evaluates every pair in FP64 and
 // records the largest FP32 error and any class mismatch (counters CNT_G32_*).  g32 > 0 needs eight wavefronts, the
 // speculative launch and a hard spherocylinder.

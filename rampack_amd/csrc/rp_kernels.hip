@@ -1371,13 +1371,13 @@ hipError_t launch_type_counts(hipStream_t s, const Proposals &pr, size_t total, 
 
 // LDS of one sweep workgroup: the stencil (cap entries), the ambiguous-candidate queues (cap + 64*waves ints),
 // own orientations, one batch of proposals and the translation table.
-// lean: the speculative sweep's own layout (spec_lds_bytes).
-size_t spec_lds_bytes(int kind, int cap, int waves, int g32);
+// lean: the speculative sweep's own layout (spec_lds_bytes, the only one that g32 changes).
+size_t spec_lds_bytes(int cap, int waves, int g32);
 
 size_t poly_lds_bytes(int waves);
 
 size_t sweep_lds_bytes(int kind, int cap, int waves, int g32, bool lean) {
-    if (lean) return kind == 2 ? poly_lds_bytes(waves) : spec_lds_bytes(kind, cap, waves, g32);
+    if (lean) return kind == 2 ? poly_lds_bytes(waves) : spec_lds_bytes(cap, waves, g32);
     const int queueInts = max(cap + WAVE * waves, (waves - 1) * GROUPED_QUEUE);
     return stencil_lds_bytes(kind, cap) + sizeof(int) * queueInts +
            sizeof(double) * (9 * OWN_CAP + 12 * MOVE_CHUNK + 81 + SWEEP_AUX) + sizeof(int) * (MOVE_CHUNK + SWEEP_AUX_I);
@@ -2339,13 +2339,13 @@ struct SpecLds {
     float *Sf, *sTf, *planF;  // guarded FP32: stencil positions (3 x cap), translation table, trial positions (3 x 32)
 };
 
-size_t spec_lds_bytes(int kind, int cap, int waves, int g32) {
-    return stencil_lds_bytes(kind, cap) + sizeof(double) * (9 * OWN_CAP + 21 + 81 + (12 + SPEC_PLAN) * SPEC_MOVES) +
-           sizeof(int) * SPEC_INTS + sizeof(uint16_t) * (kind == 0 ? 0 : waves * SPEC_QUEUE) +
+size_t spec_lds_bytes(int cap, int waves, int g32) {
+    return stencil_lds_bytes(1, cap) + sizeof(double) * (9 * OWN_CAP + 21 + 81 + (12 + SPEC_PLAN) * SPEC_MOVES) +
+           sizeof(int) * SPEC_INTS + sizeof(uint16_t) * waves * SPEC_QUEUE +
            (g32 ? sizeof(float) * (3 * (size_t)cap + 81 + 3 * SPEC_MOVES) : 0);
 }
 
-template <int KIND, int WAVES>
+template <int WAVES>
 __device__ __forceinline__ SpecLds carve_spec(double *rest, int cap) {
     SpecLds L;
     L.oo = rest;
@@ -2359,7 +2359,7 @@ __device__ __forceinline__ SpecLds carve_spec(double *rest, int cap) {
     L.cmd = L.hitOut + 1;
     L.moved = L.cmd + 1;
     L.queue = reinterpret_cast<uint16_t *>(L.moved + 4);
-    L.Sf = reinterpret_cast<float *>(L.queue + (KIND == 0 ? 0 : WAVES * SPEC_QUEUE));
+    L.Sf = reinterpret_cast<float *>(L.queue + WAVES * SPEC_QUEUE);
     L.sTf = L.Sf + 3 * cap;
     L.planF = L.sTf + 81;
     return L;
@@ -2387,7 +2387,7 @@ __device__ __forceinline__ unsigned lds_mask(const unsigned *w) {
 
 // The trial pose of this lane's move of own particle kIdx (record gi): the plan, and its word (wrap bits | inside << 3 |
 // particle << 8).  FIRST: the pose comes from the records, else from LDS.
-template <int KIND, int G32, bool FIRST>
+template <int G32, bool FIRST>
 __device__ __forceinline__ int spec_plan(const SweepParams &P, const Stencil &S, const SpecLds &L, int lane, int kIdx,
                                          int gi, int cell, const V3 &o) {
     constexpr int M = SPEC_MOVES;
@@ -2423,16 +2423,14 @@ __device__ __forceinline__ int spec_plan(const SweepParams &P, const Stencil &S,
     q[0] = inside ? npos.x : SPEC_FAR;
     q[M] = npos.y;
     q[2 * M] = npos.z;
-    if (KIND == 1) {
-        const SCFirst f = sc_first(P.k, npos, nax);
-        q[12 * M] = f.capA.x;
-        q[13 * M] = f.capA.y;
-        q[14 * M] = f.capA.z;
-        q[15 * M] = f.u.x;
-        q[16 * M] = f.u.y;
-        q[17 * M] = f.u.z;
-        q[18 * M] = f.a;
-    }
+    const SCFirst f = sc_first(P.k, npos, nax);
+    q[12 * M] = f.capA.x;
+    q[13 * M] = f.capA.y;
+    q[14 * M] = f.capA.z;
+    q[15 * M] = f.u.x;
+    q[16 * M] = f.u.y;
+    q[17 * M] = f.u.z;
+    q[18 * M] = f.a;
     if (G32) {
         L.planF[lane] = inside ? (float)(npos.x - o.x) : (float)SPEC_FAR;
         L.planF[M + lane] = (float)(npos.y - o.y);
@@ -2597,10 +2595,9 @@ __device__ __forceinline__ void spec_unit(const SpecConsts &K, const SpecLds &L,
 // move that is not in `active` has its trial position SPEC_FAR away) in units of consecutive moves, a rescan in
 // units of up to four of its moves.  PAGED: the stencil has more candidates than a queue entry names (a path of its own:
 // the page in every index costs 1 % of a sweep of 1e5 rods).
-template <int KIND, int WAVES, int G32, bool PAGED>
+template <int WAVES, int G32, bool PAGED>
 __device__ __forceinline__ void spec_scan(const SpecConsts &K, const Stencil &S, const SpecLds &L, bool translated,
                                           int nOwn, int total, unsigned active, bool whole, SpecStats &st) {
-    static_assert(KIND == 1, "the queues serve spherocylinders");
     constexpr int UNIT = G32 == 1 ? SPEC_UNIT : G32 == 0 ? SPEC_UNIT / 2 : 2;  // FP64 distances take more registers
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
@@ -2676,7 +2673,7 @@ __device__ __forceinline__ void spec_scan(const SpecConsts &K, const Stencil &S,
 }
 
 // The caller has planned the first chunk (its lanes' words in firstWord); total <= K.cap and nOwn <= OWN_CAP.
-template <int KIND, int WAVES, int G32>
+template <int WAVES, int G32>
 __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, const Stencil &S, const SpecLds &L,
                                                        bool translated, int own0, int nOwn, int total, int cell,
                                                        int firstWord, unsigned long long *clk, const V3 &o) {
@@ -2703,7 +2700,7 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
         if (wave == 0) {
             if (chunk > 0 && lane < cn) {
                 spec_proposal(P, L, lane, pbase + chunk + lane);
-                word = spec_plan<KIND, G32, false>(P, S, L, lane, P.pr.k[pbase + chunk + lane], 0, cell, o);
+                word = spec_plan<G32, false>(P, S, L, lane, P.pr.k[pbase + chunk + lane], 0, cell, o);
             }
             const unsigned in = (unsigned)__ballot(lane < cn && (word & 8));
             if (lane >= cn && lane < SPEC_MOVES) {
@@ -2732,8 +2729,8 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
             const unsigned cmd = lds_mask(L.cmd);
             if (!cmd) break;
             const unsigned long long tc0 = clk ? wall_clock64() : 0;
-            if (total <= SPEC_PAGE) spec_scan<KIND, WAVES, G32, false>(K, S, L, translated, nOwn, total, cmd, round == 0, st);
-            else spec_scan<KIND, WAVES, G32, true>(K, S, L, translated, nOwn, total, cmd, round == 0, st);
+            if (total <= SPEC_PAGE) spec_scan<WAVES, G32, false>(K, S, L, translated, nOwn, total, cmd, round == 0, st);
+            else spec_scan<WAVES, G32, true>(K, S, L, translated, nOwn, total, cmd, round == 0, st);
             __syncthreads();  // every hit of this scan is in LDS
             const unsigned long long tc1 = clk ? wall_clock64() : 0;
             if (clk) {
@@ -2760,7 +2757,7 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
                     if ((staleMask >> a) & 1) {
                         // plan the stale moves from the current poses; scan again those that stay in the cell
                         if (stale) {
-                            word = spec_plan<KIND, G32, false>(P, S, L, lane, kIdx, 0, cell, o);
+                            word = spec_plan<G32, false>(P, S, L, lane, kIdx, 0, cell, o);
                             mLo = mHi = 0;
                         }
                         tp = v3(p[0], p[M], p[2 * M]);
@@ -2778,7 +2775,7 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
                     accMask |= 1u << a;
                     moved |= 1ull << ka;
                     const double *q = L.plan + a;
-                    if (lane < (KIND == 1 ? 6 : 3)) {
+                    if (lane < 6) {
                         const int c = lane < 3 ? lane : 3 + 2 + 3 * (lane - 3);
                         S.x[lane * K.cap + ka] = q[c * M];
                     } else if (lane == 6) {
@@ -2800,18 +2797,16 @@ __device__ __forceinline__ void sweep_cell_speculative(const SweepParams &P, con
                         const V3 d = sub(p2, tp);
                         const double d2 = dot(d, d);
                         bool hit = test && d2 < K.contact2;
-                        if (KIND == 1) {
-                            const V3 a2 = v3(q[5 * M], q[8 * M], q[11 * M]);
-                            const bool close = test && !hit && d2 < K.range2 &&
-                                               !segments_apart(K.halfLen, K.skip2, d, ta, a2);
-                            if (__any(close)) {
-                                if (close) {
-                                    const V3 c2a = add(p2, scal(a2, -K.halfLen));
-                                    const V3 c2b = add(p2, scal(a2, K.halfLen));
-                                    hit = segment_distance2(v3(p[12 * M], p[13 * M], p[14 * M]),
-                                                            v3(p[15 * M], p[16 * M], p[17 * M]), p[18 * M], c2a,
-                                                            c2b) < K.contact2;
-                                }
+                        const V3 a2 = v3(q[5 * M], q[8 * M], q[11 * M]);
+                        const bool close = test && !hit && d2 < K.range2 &&
+                                           !segments_apart(K.halfLen, K.skip2, d, ta, a2);
+                        if (__any(close)) {
+                            if (close) {
+                                const V3 c2a = add(p2, scal(a2, -K.halfLen));
+                                const V3 c2b = add(p2, scal(a2, K.halfLen));
+                                hit = segment_distance2(v3(p[12 * M], p[13 * M], p[14 * M]),
+                                                        v3(p[15 * M], p[16 * M], p[17 * M]), p[18 * M], c2a,
+                                                        c2b) < K.contact2;
                             }
                         }
                         if (test) {
@@ -3742,7 +3737,7 @@ __device__ __forceinline__ void sweep_block(const SweepParams &P, const int b) {
         if (P.trace && tid == 0) trace_block(P, b, t0, nOwn, total, cell);
         return;
     } else if constexpr (LEAN != 0) {
-        const SpecLds L = carve_spec<KIND, WAVES>(rest, P.cap);
+        const SpecLds L = carve_spec<WAVES>(rest, P.cap);
         for (int i = tid; i < 81; i += NT) {
             L.sT[i] = g.T[i];
             if (G32) L.sTf[i] = (float)g.T[i];
@@ -3759,25 +3754,23 @@ __device__ __forceinline__ void sweep_block(const SweepParams &P, const int b) {
                              : v3(0, 0, 0);
             // the first wavefront plans the first moves from the global records while the others stage the stencil
             int word = 0;
-            if (WAVES == 1 || tid < WAVE) {
+            if (tid < WAVE) {
                 const int moves = P.moves > 0 ? P.moves : nOwn * P.mult;
                 if (tid < min(SPEC_MOVES, moves)) {
                     const int i = (P.moves > 0 ? cell * P.moves : own0 * P.mult) + tid, kIdx = P.pr.k[i];
                     spec_proposal(P, L, tid, i);
-                    word = spec_plan<KIND, G32, true>(P, S, L, tid, kIdx, own0 + kIdx, cell, o);
+                    word = spec_plan<G32, true>(P, S, L, tid, kIdx, own0 + kIdx, cell, o);
                 }
-            }
-            constexpr int FIRST = WAVES == 1 ? 0 : WAVE;
-            if (tid >= FIRST) {
-                stage_stencil_batched<KIND, NT - FIRST, G32 != 0>(P, S, L.sT, total, translated, L.Sf, o, FIRST);
-                for (int e = tid - FIRST; e < 9 * nOwn; e += NT - FIRST) {
+            } else {
+                stage_stencil_batched<KIND, NT - WAVE, G32 != 0>(P, S, L.sT, total, translated, L.Sf, o, WAVE);
+                for (int e = tid - WAVE; e < 9 * nOwn; e += NT - WAVE) {
                     const int c = e / nOwn, a = e - c * nOwn;
                     L.oo[c * OWN_CAP + a] = P.p.o[c][own0 + a];
                 }
             }
             if (P.phases) clk[2] = wall_clock64();
             unsigned long long *c3 = P.phases ? clk : nullptr;
-            sweep_cell_speculative<KIND, WAVES, G32>(P, S, L, translated, own0, nOwn, total, cell, word, c3, o);
+            sweep_cell_speculative<WAVES, G32>(P, S, L, translated, own0, nOwn, total, cell, word, c3, o);
         } else {
             if (P.phases) clk[2] = wall_clock64();
             // proposals in the area of the chunk's proposals and plans
@@ -3831,7 +3824,7 @@ __device__ __forceinline__ void sweep_block(const SweepParams &P, const int b) {
                 sweep_cell_staged<KIND, WAVES, true>(P, S, oo, pt, pR, pk, queue, sT, s_vote, cell, own0, nOwn, total, c3);
             else
                 sweep_cell_staged<KIND, WAVES, false>(P, S, oo, pt, pR, pk, queue, sT, s_vote, cell, own0, nOwn, total, c3);
-        } else if (WAVES >= 2 && P.pipelined == 2) {
+        } else if (WAVES >= 2 && !(KIND == 1 && WAVES == 8) && P.pipelined == 2) {  // (those run the speculative kernel)
             int *hitWords = plansI + GBUF * GPLAN_I;
             if (translated)
                 sweep_cell_grouped<KIND, WAVES, true>(P, S, oo, pt, pR, pk, queue, sT, plans, plansI, hitWords, own0,
@@ -4564,22 +4557,32 @@ bool sweep_is_lean(const PairConsts &k, int waves, int pipelined, bool counting)
     return !k.soft && !counting && ((k.kind == 2 && waves >= 4) || (waves == 8 && pipelined == 2 && k.kind == 1));
 }
 
-int sweep_occupancy(int kind, int cap, int waves) {
-    int w = waves >= 8 ? 8 : (waves >= 4 ? 4 : (waves == 2 ? 2 : 1));
-    size_t lds = sweep_lds_bytes(kind, cap, w);
+int sweep_occupancy(int kind, int cap, int waves, int g32, bool lean) {
+    const int w = waves >= 16 ? 16 : (waves >= 8 ? 8 : (waves >= 4 ? 4 : (waves == 2 ? 2 : 1)));
+    const size_t lds = sweep_lds_bytes(kind, cap, w, g32, lean);
     int blocks = 0;
-#define RP_OCC(KIND, W) hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_sweep<KIND, W, false>, WAVE * W, lds)
-    if (kind == 0) {
-        if (w == 8) RP_OCC(0, 8);
-        else if (w == 4) RP_OCC(0, 4);
-        else if (w == 2) RP_OCC(0, 2);
-        else RP_OCC(0, 1);
-    } else {
-        if (w == 8) RP_OCC(1, 8);
-        else if (w == 4) RP_OCC(1, 4);
-        else if (w == 2) RP_OCC(1, 2);
-        else RP_OCC(1, 1);
-    }
+#define RP_OCC(KIND, W, LEAN) \
+    hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_sweep<KIND, W, false, LEAN>, WAVE * W, lds)
+#define RP_OCC_W(KIND) \
+    if (w == 4) RP_OCC(KIND, 4, 0); \
+    else if (w == 2) RP_OCC(KIND, 2, 0); \
+    else RP_OCC(KIND, 1, 0);
+    if (lean && kind == 2) {
+        if (w == 16) RP_OCC(2, 16, 1);
+        else if (w == 8) RP_OCC(2, 8, 1);
+        else RP_OCC(2, 4, 1);
+    } else if (lean) {
+        if (g32 == 2) RP_OCC(1, 8, 3);
+        else if (g32 == 1) RP_OCC(1, 8, 2);
+        else RP_OCC(1, 8, 1);
+    } else if (kind == 0) {
+        if (w >= 8) RP_OCC(0, 8, 0);
+        else { RP_OCC_W(0) }
+    } else if (kind == 1) {
+        if (w >= 8) RP_OCC(1, 8, 0);
+        else { RP_OCC_W(1) }
+    } else { RP_OCC_W(2) }
+#undef RP_OCC_W
 #undef RP_OCC
     return blocks;
 }
@@ -4612,8 +4615,7 @@ hipError_t launch_sweep(hipStream_t s, const SweepParams &sp, int waves, Timed t
     int w = waves >= 16 ? 16 : (waves >= 8 ? 8 : (waves >= 4 ? 4 : (waves == 2 ? 2 : 1)));
     if (w == 16 && (sp.k.kind != 2 || sp.counting || sp.fixMode)) w = 8;  // sixteen only for the polysphere sweep
     if (w == 8 && (sp.k.soft || sp.counting)) w = 4;  // eight only for the hard sweeps
-    // the lean kernels run spherocylinders only: their first launch on spheres (eight wavefronts forced onto sparse
-    // stencils) faulted the GPU and the cause is not found, so spheres keep the general kernel
+    // the guarded scan is the speculative spherocylinder kernel's
     if (g32 && (w != 8 || sp.pipelined != 2 || sp.fixMode || sp.k.kind != 1)) return hipErrorInvalidValue;
     const bool lean = !sp.fixMode && sweep_is_lean(sp.k, w, sp.pipelined, sp.counting != 0);
     size_t lds = sweep_lds_bytes(sp.k.kind, sp.cap, w, g32, lean);
