@@ -109,7 +109,7 @@ class AutotuneEntry(ctypes.Structure):
 
 
 AUTOTUNE_MAX = 8
-SCHEDULES = ("plain", "pipelined", "grouped")
+SCHEDULES = ("plain", "pipelined", "grouped")  # "grouped" on eight wavefronts of spherocylinders: the speculative sweep
 
 
 class Observables(ctypes.Structure):

@@ -2313,7 +2313,7 @@ __device__ __forceinline__ void sweep_cell_grouped(const SweepParams &P, const S
 // unit); an accepted move costs about 1.2 us of one wavefront's latency.  Per workgroup on 1e5 rods (L/D 5, packing
 // fraction 0.45): staging 3.5 us, first scan 11.4, 1.2 rescans 2.8, 4.8 accepted moves 5.6; the groups of four moves
 // with a barrier each that this replaces took 52 us for the same moves.  100 cycles: 67.0 -> 51.5 ms on 1e5 rods,
-// 43.9 -> 38.6 ms on 8 000 (guarded), 50 cycles on 1e6: 414 -> 207 ms.
+// 43.9 -> 37.8 ms on 8 000 (guarded), 50 cycles on 1e6: 414 -> 208 ms.
 constexpr int SPEC_MOVES = 32;     // moves per chunk
 constexpr int SPEC_PLAN = 19;      // doubles per plan: npos 3, NO 9, capA 3, u 3, a 1 (component c of move m at c * 32 + m)
 constexpr int SPEC_UNIT = 8;       // moves per unit of the first scan
