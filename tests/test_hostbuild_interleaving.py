@@ -40,13 +40,13 @@ def run_case(lib, *args, **env):
     assert "case passed" in res.stdout
 
 
-@pytest.mark.parametrize("order, samplers, precision", [("lowest", 1, 0), ("highest", 1, 1), ("3", 2, 0), ("lowest", 2, 1)])
+@pytest.mark.parametrize("order, samplers, precision", [("lowest", 1, 0), ("lowest", 1, 1), ("highest", 1, 0), ("3", 2, 0)])
 def test_rods_follow_one_wavefront(host_lib, order, samplers, precision):
     """About 50 moves per cell and sampler: two or four chunks."""
     run_case(host_lib, "rods", "28,28,4", "1.2,1.2,6.3", 0.1, samplers, precision, 2, EMU_SCHED_SEED=order)
 
 
-@pytest.mark.parametrize("order", ["lowest", "highest", "3"])
+@pytest.mark.parametrize("order", ["lowest", "3"])
 def test_chains_follow_one_wavefront(host_lib, order):
     run_case(host_lib, "chains", 16, "20,20,2", "1.25,1.25,16.8", 0.2, 4, 1, EMU_SCHED_SEED=order)
 
